@@ -118,7 +118,7 @@ struct Scratch {
   uint64_t slab;     // bytes per wave
   // offsets inside a slab
   uint64_t o_cmap, o_bm0, o_bm1, o_L, o_Lp, o_T, o_kL, o_U, o_Ucnt, o_C, o_kC, o_R, o_fr,
-      o_dom, o_arena, o_ctx;
+      o_save, o_arena, o_ctx;
   uint64_t arena_bytes, ctx_bytes;  // ctx_bytes: per context slot
   uint32_t ctx_slots;                // context slots per wave
   uint32_t nW0, nW1;
@@ -195,6 +195,12 @@ struct Counters {
   LdsCount blist;  // bytes of the bitset lists pushes read and write, CSR bytes of task roots
 };
 constexpr int kCounters = (int)(sizeof(Counters) / sizeof(LdsCount));
+
+}  // namespace mbe
+
+#include "small_dfs.hpp"
+
+namespace mbe {
 
 // Per-graph result counters of a batch (u64 each, kPerGraph per graph).
 enum PerGraph : int {
@@ -576,7 +582,6 @@ struct WaveMem {
   uint32_t* R;     // closure of L
   Frame* fr;       // DFS frames (slab; the first kLdsFrames live in fr_lds)
   Frame* fr_lds;   // DFS frames in LDS
-  uint64_t* dom;   // dominator bitsets of reduce_list (kMaxDom x kMaxW)
   char* arena;     // HBM list arena
   uint64_t arena_bytes;
   char* lds;       // LDS list arena
@@ -585,6 +590,7 @@ struct WaveMem {
   int64_t* s_start;// 64 i64 in LDS
   const DevGraph* g;  // graph of the current unit of work (set per unit)
   uint64_t deadline;  // wall clock past which this wave stops (with a budget)
+  SmallCall* sc;      // call block of small_dfs, in LDS
 };
 
 // Whether p lies in this wave's LDS list arena.
@@ -661,7 +667,6 @@ __device__ __forceinline__ WaveMem wave_mem(const Params& P, uint64_t gw, char* 
   m.R = (uint32_t*)(b + S.o_R);
   m.fr = (Frame*)(b + S.o_fr);
   m.fr_lds = fr_lds;
-  m.dom = (uint64_t*)(b + S.o_dom);
   m.arena = b + S.o_arena;
   m.arena_bytes = S.arena_bytes;
   m.lds = lds;
@@ -695,6 +700,31 @@ __device__ __forceinline__ uint64_t list_reserve(const Params& P, uint64_t words
     }
   }
   return uni64(at);
+}
+
+// Whether lists of at most 64 one-word entries go to small_dfs.  It relies on
+// ordered lists (dom_skip), reduces every list, and neither lists bicliques nor
+// counts bytes: those runs stay on the general stack machine.
+__device__ __forceinline__ bool use_small(const Params& P) {
+  return P.dom_skip && !P.list && !P.count_bytes && P.reduce_min <= 0;
+}
+
+// The call block's fields that hold for the whole kernel (once per wave).
+__device__ __forceinline__ void small_setup(const Params& P, const WaveMem& m, uint64_t gw) {
+  const unsigned long long n_roots = roots_total(P.s);
+  if (lane_id() == 0) {
+    auto* sc = as_lds(m.sc);
+    sc->root_next = P.s.root_next;
+    sc->queued = P.s.queued;
+    sc->n_roots = n_roots;
+    sc->deadline = P.budget != 0 ? m.deadline : 0;
+    sc->save = (uint32_t*)(P.w.base + gw * P.w.slab + P.w.o_save);
+    sc->share_queue = P.share_queue;
+    sc->share_len = P.late_share > 0 ? (uint32_t)P.late_share : 0u;
+    sc->dom_k = (uint32_t)(P.dom_k < kMaxDom ? (P.dom_k > 0 ? P.dom_k : 0) : kMaxDom);
+    sc->prune = P.prune != 0;
+  }
+  wave_mem_wait();
 }
 
 // ---------------------------------------------------------------------------
@@ -792,29 +822,42 @@ __device__ __forceinline__ PassOut push_pass(Rec<W>* recs, uint32_t len, const u
   bool dead = false;
   uint64_t absorbed = 0, best_next = ~0ull, best_child = ~0ull;
   uint32_t clen = 0, cbranch = 0;
+  // the next chunk is loaded before this one's entries are written: the child
+  // list is another array, and a prune mark only touches the chunk in hand
+  Rec<W> nx;
+  auto load = [&](uint32_t k) {
+    nx.minidx = kNone;
+    nx.rep = kNone;
+    nx.ksum = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) nx.a[w] = 0;
+    if (k < len) {
+      if constexpr (LDS_IN) {
+        const auto* q = as_lds(recs) + k;
+        nx.minidx = q->minidx;
+        nx.rep = q->rep;
+        nx.ksum = q->ksum;
+#pragma unroll
+        for (int w = 0; w < W; ++w) nx.a[w] = q->a[w];
+      } else {
+        nx.minidx = rd<LIST_REMOTE>(&recs[k].minidx);
+        nx.rep = rd<LIST_REMOTE>(&recs[k].rep);
+        nx.ksum = rd<LIST_REMOTE>(&recs[k].ksum);
+#pragma unroll
+        for (int w = 0; w < W; ++w) nx.a[w] = rd<LIST_REMOTE>(&recs[k].a[w]);
+      }
+    }
+  };
+  load(lane);
   for (uint32_t base = 0; base < len; base += kWave) {
     const uint32_t k = base + lane;
     const bool valid = k < len;
-    uint32_t mi = kNone, rep = kNone;
-    uint64_t ks = 0, ae[W];
+    const uint32_t mi = nx.minidx, rep = nx.rep;
+    const uint64_t ks = nx.ksum;
+    uint64_t ae[W];
 #pragma unroll
-    for (int w = 0; w < W; ++w) ae[w] = 0;
-    if (valid) {
-      if constexpr (LDS_IN) {
-        const auto* q = as_lds(recs) + k;
-        mi = q->minidx;
-        rep = q->rep;
-        ks = q->ksum;
-#pragma unroll
-        for (int w = 0; w < W; ++w) ae[w] = q->a[w];
-      } else {
-        mi = rd<LIST_REMOTE>(&recs[k].minidx);
-        rep = rd<LIST_REMOTE>(&recs[k].rep);
-        ks = rd<LIST_REMOTE>(&recs[k].ksum);
-#pragma unroll
-        for (int w = 0; w < W; ++w) ae[w] = rd<LIST_REMOTE>(&recs[k].a[w]);
-      }
-    }
+    for (int w = 0; w < W; ++w) ae[w] = nx.a[w];
+    load(k + kWave);
     // maximality first, for the whole chunk: a chunk that shows the node is
     // non-maximal writes none of its child entries
     bool sub = valid, zero = true, inside = valid;
@@ -1111,6 +1154,149 @@ __device__ __forceinline__ bool publish_list(const Params& P, uint64_t gw, uint3
   return true;
 }
 
+// Publish a node of small_dfs (at most 64 entries, one per lane) as this wave's
+// context and push one item per entry still to be pushed: publish_list for a
+// list in registers.  Entries are renumbered by position, which keeps their
+// order, all that a push looks at.
+__device__ __forceinline__ bool publish_small(const Params& P, uint64_t gw, uint32_t ctx,
+                                              uint32_t gid, uint32_t nL, uint64_t a0, uint64_t ks,
+                                              uint64_t key, uint64_t L, uint64_t alive,
+                                              uint64_t push, uint64_t todo, uint64_t sumR) {
+  const uint32_t lane = lane_id();
+  const Sched& s = P.s;
+  const uint32_t len = (uint32_t)__popcll(alive), n_items = (uint32_t)__popcll(todo);
+  if (ctx_bytes<1>(nL, 0, len) > P.w.ctx_bytes) return false;
+  const uint32_t ne = (n_items + kItemsPerEntry - 1) / kItemsPerEntry;
+  CtxHdr* h = ctx_hdr(P, ctx);
+  Rec<1>* recs;
+  TaskArrays ta;
+  ctx_arrays<1>(h, nL, 0, len, recs, ta);
+  const uint32_t pos = lanes_below(alive);
+  if (lane_bit(alive)) {
+    st_dev(&recs[pos].minidx, pos);
+    st_dev(&recs[pos].rep, lane_bit(push) ? pos : kNone);
+    st_dev(&recs[pos].ksum, ks);
+    st_dev(&recs[pos].a[0], a0 & L);
+  }
+  if (lane < nL) st_dev((uint64_t*)ta.kL + lane, key);
+  if (lane == 0) {
+    st_dev(&h->sumR0, sumR);
+    st_dev(&h->nbits, (uint32_t)__popcll(L));
+    st_dev(&h->nL, nL);
+    st_dev(&h->nC, 0u);
+    st_dev(&h->len, len);
+    st_dev(&h->W, 1u);
+    st_dev(&h->gid, gid);
+    st_dev(&h->refs, (unsigned long long)n_items);
+  }
+  wave_drain();
+  uint32_t sh = 0;
+  unsigned long long start = 0;
+  if (!queue_reserve(s, (uint32_t)(gw & (kShards - 1)), ne, sh, start)) {
+    if (lane == 0) st_dev(&h->refs, 0ull);
+    return false;
+  }
+  if (lane == 0)
+    __hip_atomic_fetch_add(s.work_left, (unsigned long long)ne, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+  graph_work(P, gid, (long long)ne);
+  // item j (the j-th bit of todo) goes to entry j / 15, slot j % 15
+  if (lane_bit(todo)) {
+    const uint32_t j = lanes_below(todo);
+    const unsigned long long at = start + j / kItemsPerEntry;
+    const uint64_t slot = slot_of(s, sh, at);
+    uint32_t* e = s.q + slot * kEntryWords;
+    const uint32_t i = j % kItemsPerEntry;
+    // a slot is free once its sequence number says so: every lane waits for its own
+    while (ld_dev(s.qseq + slot) != at) __builtin_amdgcn_s_sleep(1);
+    if (i == 0) {
+      const uint32_t left = n_items - j;
+      st_dev(e + 0, kItemKind | (left < (uint32_t)kItemsPerEntry ? left : (uint32_t)kItemsPerEntry));
+      st_dev(e + 1, ctx);
+    }
+    st_dev(e + 2 + 2 * i, pos);
+    st_dev(e + 3 + 2 * i, pos);
+  }
+  wave_drain();
+  if (lane < ne) st_dev(s.qseq + slot_of(s, sh, start + lane), start + lane + 1);
+  wave_drain();
+  if (lane == 0)
+    __hip_atomic_fetch_add(s.queued, (unsigned long long)ne, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+// The subtree of a node whose list is in the lanes (see small_dfs): `todo`
+// the entries to push, `push` those that may be pushed in it, nL the number of
+// L indices the bitsets range over.  Handles what the stack machine leaves to
+// its caller: sharing a node with other waves, and the deadline.
+__device__ __forceinline__ void run_small(const Params& P, const WaveMem& m, uint64_t gw,
+                                          uint32_t nL, uint64_t a0, uint64_t ks, uint64_t key,
+                                          uint64_t alive, uint64_t push, uint64_t todo,
+                                          uint64_t sumR, Counters& ctr) {
+  if (todo == 0) return;
+  const uint32_t gid = graph_id(P, m);
+  auto* sc = as_lds(m.sc);
+  if (lane_id() == 0) {
+    sc->swapped = m.g->swapped;
+    sc->L = ~0ull;
+    sc->alive = alive;
+    sc->push = push;
+    sc->todo = todo;
+    sc->sumR = sumR;
+  }
+  wave_mem_wait();
+  uint32_t how = SMALL_START;
+  for (;;) {
+    const uint32_t st = uni(P.profile ? small_dfs<true>(sc, &ctr, nL, how, a0, ks, key)
+                                      : small_dfs<false>(sc, &ctr, nL, how, a0, ks, key));
+    if (st == SMALL_DONE) return;
+    if (st == SMALL_CUT) {
+      ctr.abandoned++;
+      graph_work(P, gid, 1);  // never finished: the graph stays incomplete
+      return;
+    }
+    how = SMALL_RESUME;
+    const uint32_t cx = free_ctx(P, gw);
+    if (cx != kNone &&
+        publish_small(P, gw, cx, gid, nL, a0, ks, key, uni64(sc->sh_L), uni64(sc->sh_alive),
+                      uni64(sc->sh_push), uni64(sc->sh_todo), uni64(sc->sh_sumR))) {
+      how = SMALL_RESUME_SHARED;
+      ctr.splits++;
+      ctr.publishes++;
+      ctr.late++;
+    }
+  }
+}
+
+// The same for a list in memory (len <= 64 ordered one-word entries, with skip
+// marks), in this wave's arenas; kL: the hash keys of its L indices.
+__device__ __forceinline__ void run_small_list(const Params& P, const WaveMem& m, uint64_t gw,
+                                               uint32_t nL, const uint64_t* kL,
+                                               const Rec<1>* recs, uint32_t len, uint64_t sumR,
+                                               Counters& ctr) {
+  const uint32_t lane = lane_id();
+  uint32_t mi = 0, rp = kNone;
+  uint64_t ks = 0, a0 = 0, key = 0;
+  if (in_lds(m, recs)) {
+    if (lane < len) {
+      const auto* q = as_lds(recs) + lane;
+      mi = q->minidx;
+      rp = q->rep;
+      ks = q->ksum;
+      a0 = q->a[0];
+    }
+  } else if (lane < len) {
+    mi = recs[lane].minidx;
+    rp = recs[lane].rep;
+    ks = recs[lane].ksum;
+    a0 = recs[lane].a[0];
+  }
+  if (lane < nL) key = in_lds(m, kL) ? as_lds(kL)[lane] : kL[lane];
+  const uint64_t push = ballot(rp != kNone), skip = ballot((mi & kSkip) != 0);
+  run_small(P, m, gw, nL, a0, ks, key, ballot(lane < len), push, push & ~skip, sumR, ctr);
+}
+
 // Merge the entries of a list (len entries at crec) whose bitsets are
 // identical: minidx and rep by minimum, ksum by sum, in place.  Open
 // addressing in a table taken from the arenas (LDS first); a slot's identity
@@ -1401,31 +1587,37 @@ __device__ __forceinline__ uint32_t reduce_list(const Params& P, const WaveMem& 
   }
   const uint32_t minrep = (uint32_t)(best >> 32);
   lds_flat_fence();  // a list in LDS is reached below through generic pointers
-  // dominators: K rounds of a maximum over key = (popcount + 1) << 20 | ~pos
-  // among the excluded entries, each round below the previous maximum
-  uint32_t dpos[kMaxDom];
-  int nd = 0;
-  uint32_t prev = 0xFFFFFFFFu;
-  for (int r = 0; r < K; ++r) {
-    uint32_t kb = 0;
-    for (uint32_t base = 0; base < len; base += kWave) {
-      const uint32_t i = base + lane;
-      if (i < len && recs[i].rep == kNone && (recs[i].minidx & ~kSkip) < minrep) {
-        uint32_t pc = 0;
+  // dominators: every lane keeps its two largest keys = (popcount + 1) << 20 |
+  // ~pos among the excluded entries of one pass over the list, and K maxima
+  // over the wave pick from those (a third of one lane is never tried; a pass
+  // per dominator, which would find it, cost eight times the reads)
+  uint32_t k1 = 0, k2 = 0;
+#pragma unroll 4
+  for (uint32_t i = lane; i < len; i += kWave) {
+    if (recs[i].rep == kNone && (recs[i].minidx & ~kSkip) < minrep) {
+      uint32_t pc = 0;
 #pragma unroll
-        for (int w = 0; w < W; ++w) pc += __popcll(recs[i].a[w]);
-        const uint32_t k = ((pc + 1) << 20) | (0xFFFFFu - i);
-        if (k < prev && k > kb) kb = k;
-      }
+      for (int w = 0; w < W; ++w) pc += __popcll(recs[i].a[w]);
+      const uint32_t k = ((pc + 1) << 20) | (0xFFFFFu - i);
+      k2 = k > k1 ? k1 : k > k2 ? k : k2;
+      k1 = k > k1 ? k : k1;
     }
-    const uint32_t mx = wave_max_u32(kb);
-    if (mx == 0) break;
-    const uint32_t pd = 0xFFFFFu - (mx & 0xFFFFFu);
-    // keep the dominator's bitset: compaction may overwrite its entry
-    if (lane < (uint32_t)W) m.dom[nd * kMaxW + lane] = recs[pd].a[lane];
-    dpos[nd++] = pd;
-    prev = mx;
   }
+  // lane d holds dominator d: position, then bitset (one gather for all)
+  uint32_t dposv = 0;
+  uint64_t dom[W];
+  int nd = 0;
+  for (; nd < K; ++nd) {
+    const uint32_t mx = wave_max_u32(k1);
+    if (mx == 0) break;
+    dposv = write_lane(dposv, 0xFFFFFu - (mx & 0xFFFFFu), (uint32_t)nd);
+    if (k1 == mx) {
+      k1 = k2;
+      k2 = 0;
+    }
+  }
+#pragma unroll
+  for (int w = 0; w < W; ++w) dom[w] = lane < (uint32_t)nd ? recs[dposv].a[w] : 0;
   lds_flat_fence();
   if (nd == 0 && !P.dom_skip) {
     if (P.profile) ctr.c_reduce += cycles() - tr;
@@ -1433,29 +1625,36 @@ __device__ __forceinline__ uint32_t reduce_list(const Params& P, const WaveMem& 
   }
   uint32_t out = 0, nbr = 0, ndrop = 0, nskip = 0;
   uint64_t nb = ~0ull;
+  // compaction writes only below the chunk it reads, so the next chunk is
+  // loaded before this one is written
+  Rec<W> nx;
+  auto load = [&](uint32_t i) {
+    nx.minidx = kNone;
+    nx.rep = kNone;
+    nx.ksum = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) nx.a[w] = 0;
+    if (i < len) nx = recs[i];
+  };
+  load(lane);
   for (uint32_t base = 0; base < len; base += kWave) {
     const uint32_t i = base + lane;
     const bool valid = i < len;
-    uint32_t mi = kNone, rp = kNone;
-    uint64_t ks = 0, a[W];
+    const uint32_t mi = valid ? nx.minidx & ~kSkip : kNone, rp = nx.rep;
+    const uint64_t ks = nx.ksum;
+    uint64_t a[W];
 #pragma unroll
-    for (int w = 0; w < W; ++w) a[w] = 0;
-    if (valid) {
-      mi = recs[i].minidx & ~kSkip;
-      rp = recs[i].rep;
-      ks = recs[i].ksum;
-#pragma unroll
-      for (int w = 0; w < W; ++w) a[w] = recs[i].a[w];
-    }
+    for (int w = 0; w < W; ++w) a[w] = nx.a[w];
+    load(i + kWave);
     const bool excl = valid && rp == kNone && mi < minrep;
     const bool push = valid && rp != kNone;
     bool drop = false, sk = push && mi < rp;
     for (int d = 0; d < nd; ++d) {
-      const uint32_t pd = dpos[d];
+      const uint32_t pd = read_lane(dposv, (uint32_t)d);
       bool inside = true, eq = true;
 #pragma unroll
       for (int w = 0; w < W; ++w) {
-        const uint64_t dw = m.dom[d * kMaxW + w];
+        const uint64_t dw = read_lane64(dom[w], (uint32_t)d);
         inside = inside && (a[w] & ~dw) == 0;
         eq = eq && a[w] == dw;
       }
@@ -1573,6 +1772,12 @@ __device__ __forceinline__ bool child_node(const Params& P, const WaveMem& m, ui
           hbm_top = sh;
           return false;
         }
+        if (use_small(P) && dlen <= (uint32_t)kWave) {
+          run_small_list(P, m, gw, nb, kLc, dst, dlen, sumR, ctr);
+          lds_top = sl;
+          hbm_top = sh;
+          return false;
+        }
         TaskArrays tc{kLc, ta.C};
         bool shared = false;
         const uint32_t cx = P.share && (uint64_t)dlen * dcb >= (uint64_t)P.share_work
@@ -1617,6 +1822,12 @@ __device__ __forceinline__ bool child_node(const Params& P, const WaveMem& m, ui
   }
   clen = reduce_list<W>(P, m, crec, clen, best_child, cbranch, ctr);
   if (cbranch == 0) return false;  // every push of the node is known to be non-maximal
+  if constexpr (W == 1 && !KL_R) {
+    if (use_small(P) && clen <= (uint32_t)kWave) {
+      run_small_list(P, m, gw, nL, ta.kL, crec, clen, sumR, ctr);
+      return false;
+    }
+  }
   const uint32_t cx = P.share && !P.list && (uint64_t)clen * cbranch >= (uint64_t)P.share_work
                           ? share_wanted(P, gw, nL, nC, clen, W)
                           : kNone;
@@ -1876,6 +2087,30 @@ __device__ __forceinline__ void run_items_w(const Params& P, const WaveMem& m, C
   R_t* recs;
   TaskArrays rta;
   ctx_arrays<W>(h, nL, nC, len, recs, rta);
+  if constexpr (W == 1) {
+    if (use_small(P) && len <= (uint32_t)kWave) {
+      // the whole entry at once: its items are the pushes left at the node
+      const uint32_t lane = lane_id();
+      uint64_t t0 = P.profile ? cycles() : 0;
+      uint32_t rp = kNone;
+      uint64_t ks = 0, a0 = 0, key = 0;
+      if (lane < len) {
+        rp = ld_dev(&recs[lane].rep);
+        ks = ld_dev(&recs[lane].ksum);
+        a0 = ld_dev(&recs[lane].a[0]);
+      }
+      if (lane < nL) key = ld_dev(rta.kL + lane);
+      uint64_t todo = 0;
+      for (uint32_t it = 0; it < cnt; ++it) todo |= 1ull << read_lane(word, 2 + 2 * it);
+      run_small(P, m, gw, nL, a0, ks, key, ballot(lane < len), ballot(rp != kNone), todo, sumR0,
+                ctr);
+      if (lane == 0)
+        __hip_atomic_fetch_add(&h->refs, (unsigned long long)(-(long long)cnt), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+      phase(ctr, P.profile, 5, t0);
+      return;
+    }
+  }
   // the hash keys of L, read at every maximal push below: a local copy at
   // the bottom of the arenas (LDS when it fits)
   uint32_t lds0 = 0;
@@ -2069,6 +2304,14 @@ __device__ __forceinline__ void enumerate_task(const Params& P, const WaveMem& m
     ctr.splits++;
     phase(ctr, P.profile, 6, t0);
     return;
+  }
+  if constexpr (Wt == 1) {
+    if (use_small(P) && len <= (uint32_t)kWave) {
+      phase(ctr, P.profile, 4, t0);
+      run_small_list(P, m, gw, nL, m.kL, brec, len, sumR, ctr);
+      phase(ctr, P.profile, 5, t0);
+      return;
+    }
   }
   // the hash keys of L, read at every maximal push: into LDS when small
   const uint64_t* kL = m.kL;

@@ -41,6 +41,9 @@ void mbe_persistent(Params P) {
     }
   }
   m.deadline = dl;
+  __shared__ SmallCall s_small[WAVES];
+  m.sc = &s_small[wv];
+  small_setup(P, m, gw);
   __shared__ Counters s_ctr[WAVES];
   Counters& c = s_ctr[wv];
   for (int i = (int)lane_id(); i < kCounters; i += kWave) as_lds(&c.maximal)[i].v = 0;

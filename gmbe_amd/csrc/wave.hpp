@@ -39,6 +39,18 @@ __device__ __forceinline__ uint64_t read_lane64(uint64_t x, uint32_t l) {
   uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), l);
   return ((uint64_t)hi << 32) | lo;
 }
+// x with lane l's value replaced by the uniform v (the intrinsic has no
+// builtin in this compiler)
+__device__ uint32_t llvm_writelane(uint32_t v, uint32_t l, uint32_t x) __asm(
+    "llvm.amdgcn.writelane.i32");
+__device__ __forceinline__ uint32_t write_lane(uint32_t x, uint32_t v, uint32_t l) {
+  return llvm_writelane(v, l, x);
+}
+__device__ __forceinline__ uint64_t write_lane64(uint64_t x, uint64_t v, uint32_t l) {
+  const uint32_t lo = write_lane((uint32_t)x, (uint32_t)v, l);
+  const uint32_t hi = write_lane((uint32_t)(x >> 32), (uint32_t)(v >> 32), l);
+  return ((uint64_t)hi << 32) | lo;
+}
 __device__ __forceinline__ uint32_t shfl_xor32(uint32_t x, int m) {
   return (uint32_t)__shfl_xor((int)x, m, kWave);
 }
@@ -68,6 +80,13 @@ __device__ __forceinline__ uint32_t wave_incl_scan32(uint32_t x) {
     if (l >= (uint32_t)d) x += y;
   }
   return x;
+}
+// c & plane where that is not empty, else c (uniform masks): one and, one select
+// on its condition code
+__device__ __forceinline__ uint64_t narrow(uint64_t c, uint64_t plane) {
+  uint64_t r;
+  asm("s_and_b64 %0, %1, %2\n\ts_cselect_b64 %0, %0, %1" : "=&s"(r) : "s"(c), "s"(plane) : "scc");
+  return r;
 }
 __device__ __forceinline__ int first_lane(uint64_t m) { return __builtin_ctzll(m); }
 // This lane's bit of a uniform lane mask (32-bit shifts only).
@@ -122,6 +141,24 @@ __device__ __forceinline__ uint64_t wave_sum_u64(uint64_t x) {
   const uint32_t lo = __builtin_amdgcn_readlane((uint32_t)x, 63);
   const uint32_t hi = __builtin_amdgcn_readlane((uint32_t)(x >> 32), 63);
   return ((uint64_t)hi << 32) | lo;
+}
+
+// Exclusive or over the wave by the same steps.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t dpp_xor64(uint64_t x) {
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWS, 0xf, false);
+  const uint32_t hi =
+      (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), CTRL, ROWS, 0xf, false);
+  return x ^ (((uint64_t)hi << 32) | lo);
+}
+__device__ __forceinline__ uint64_t wave_xor_u64(uint64_t x) {
+  x = dpp_xor64<0x111, 0xf>(x);
+  x = dpp_xor64<0x112, 0xf>(x);
+  x = dpp_xor64<0x114, 0xf>(x);
+  x = dpp_xor64<0x118, 0xf>(x);
+  x = dpp_xor64<0x142, 0xa>(x);
+  x = dpp_xor64<0x143, 0xc>(x);
+  return read_lane64(x, 63);
 }
 
 // A generic pointer known to address LDS, as an LDS pointer: accesses through

@@ -250,7 +250,8 @@ int gmbe_finder_exit_times(const gmbe_finder* f, double* out, size_t cap, size_t
  * buffer); [12] list entries and [13] pushes in one-word-bitset lists;
  * [14] cycles of the final wait (a wave with nothing left to do);
  * [15..18] cycles inside the stack machine spent in push passes, twin
- * merges, bitset re-indexing and context publishing; [19] contexts
+ * merges, bitset re-indexing and context publishing (of lists of more than 64
+ * entries or one bitset word: shorter ones are one register machine); [19] contexts
  * published, [20] twin merges; [21] subtrees abandoned at the deadline;
  * [22] frames handed over by late sharing; [23] cycles spent reducing
  * lists, [24] excluded entries dropped, [25] pushes marked non-maximal;
