@@ -19,7 +19,10 @@ struct Engine {
 struct DeviceGraph {
   uint32_t nU = 0, nV = 0, dmaxV = 0;
   uint64_t E = 0;
+  uint64_t max_cand = 0;  // no 2-hop neighbourhood of a V vertex is larger
+  uint64_t cost = 0;      // edges of all 2-hop passes: sum over V of sum over N(v) of deg(u)
   int swapped = 0;
+  char* block = nullptr;  // the allocation the arrays below lie in
   int64_t *v_off = nullptr, *u_off = nullptr;
   uint32_t *v_adj = nullptr, *u_adj = nullptr;
   uint64_t *kUd = nullptr, *kVd = nullptr;
@@ -69,6 +72,8 @@ hipError_t launch_reset_ctx(hipStream_t st, const mbe::Params& P, unsigned long 
 hipError_t launch_init_left(hipStream_t st, const mbe::Params& P, unsigned long long n);
 hipError_t launch_fill(hipStream_t st, unsigned long long* p, unsigned long long n,
                        unsigned long long v);
+// Zero the count maps and bitmaps of n fresh slabs.
+hipError_t launch_zero_slabs(hipStream_t st, const mbe::Scratch& w, unsigned long long n);
 // Control block for a new launch: zero, then work_left = n_roots; with
 // keep_deadline the run's deadline word stays (a later launch of one run).
 hipError_t launch_ctl_start(hipStream_t st, unsigned long long* ctl, unsigned long long n_roots,

@@ -42,6 +42,40 @@ __global__ void init_queue(unsigned long long* seq, unsigned long long cap) {
     seq[i] = i & (cap - 1);
 }
 
+// Everything a finder's run starts from, in one launch: the control block
+// (zero but the outstanding work), the result counters, the queue's sequence
+// numbers, the context slots and the graph table.  Four launches and three
+// copies before it took 40 us of a 220 us run on the smallest graphs.
+__global__ void run_start(Params P, unsigned long long* ctl, unsigned long long words,
+                          unsigned long long wl, unsigned long long n_roots,
+                          unsigned long long n_ctx, DevGraph* gt, DevGraph g) {
+  const unsigned long long t = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x,
+                           step = (unsigned long long)gridDim.x * blockDim.x;
+  if (t == 0) *gt = g;
+  for (unsigned long long i = t; i < words; i += step) ctl[i] = i == wl ? n_roots : 0ull;
+  for (unsigned long long i = t; i < A_COUNT; i += step) P.acc[i] = 0ull;
+  for (unsigned long long i = t; i < P.s.qcap * kShards; i += step)
+    P.s.qseq[i] = i & (P.s.qcap - 1);
+  for (unsigned long long i = t; i < n_ctx; i += step) ctx_hdr(P, i)->refs = 0ull;
+}
+
+// The control words and counters the host reads after a pass, into pinned host
+// memory (one small kernel instead of two copies through a staging buffer).
+__global__ void run_result(const unsigned long long* ctl, unsigned long long stride, int n_ctl,
+                           const unsigned long long* acc, unsigned long long* out) {
+  for (int i = threadIdx.x; i < n_ctl + (int)A_COUNT; i += blockDim.x)
+    out[i] = i < n_ctl ? ctl[(unsigned long long)i * stride] : acc[i - n_ctl];
+}
+
+// Zero what must be zero in fresh slabs: the count map and the bitmaps, which
+// lead every slab (words u64 of each; the rest is written before it is read).
+__global__ void zero_slabs(char* base, unsigned long long slab, unsigned long long words,
+                           unsigned long long n) {
+  for (unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x;
+       i < n * words; i += (unsigned long long)gridDim.x * blockDim.x)
+    ((unsigned long long*)(base + i / words * slab))[i % words] = 0ull;
+}
+
 // Fill n u64 words with v.
 __global__ void fill_u64(unsigned long long* p, unsigned long long n, unsigned long long v) {
   for (unsigned long long i = (unsigned long long)blockIdx.x * blockDim.x + threadIdx.x; i < n;
@@ -141,6 +175,12 @@ hipError_t launch_fill(hipStream_t st, unsigned long long* p, unsigned long long
   hipLaunchKernelGGL(mbe::fill_u64, dim3((unsigned)blocks), dim3(256), 0, st, p, n, v);
   return hipGetLastError();
 }
+hipError_t launch_zero_slabs(hipStream_t st, const mbe::Scratch& w, unsigned long long n) {
+  // cmap, bm0 and bm1 are the first three arrays of a slab (scratch_layout)
+  hipLaunchKernelGGL(mbe::zero_slabs, dim3(1024), dim3(256), 0, st, w.base,
+                     (unsigned long long)w.slab, (unsigned long long)w.o_L / 8, n);
+  return hipGetLastError();
+}
 hipError_t launch_ctl_start(hipStream_t st, unsigned long long* ctl, unsigned long long n_roots,
                             bool keep_deadline) {
   hipLaunchKernelGGL(mbe::ctl_start, dim3(1), dim3(256), 0, st, ctl, kCtlWords,
@@ -181,37 +221,51 @@ int DeviceGraph::upload(const gmbe_graph& g) {
   E = g.E;
   swapped = g.swapped;
   dmaxV = 0;
-  for (uint32_t v = 0; v < g.nV; ++v)
+  max_cand = 0;
+  cost = 0;
+  for (uint32_t v = 0; v < g.nV; ++v) {
     dmaxV = std::max<uint32_t>(dmaxV, (uint32_t)(g.v_off[v + 1] - g.v_off[v]));
+    uint64_t c = 0;
+    for (int64_t e = g.v_off[v]; e < g.v_off[v + 1]; ++e)
+      c += (uint64_t)(g.u_off[g.v_adj[e] + 1] - g.u_off[g.v_adj[e]]);
+    cost += c;
+    max_cand = std::max(max_cand, std::min<uint64_t>(c, g.nV));
+  }
   std::vector<uint64_t> kU, kV;
   hash_keys(g, kU, kV);
-  size_t b_voff = (size_t)(nV + 1) * 8, b_uoff = (size_t)(nU + 1) * 8;
-  size_t b_adj = (size_t)std::max<uint64_t>(E, 1) * 4;
-  size_t b_kU = (size_t)std::max<uint32_t>(nU, 1) * 8, b_kV = (size_t)std::max<uint32_t>(nV, 1) * 8;
-  HIP_TRY(hipMalloc(&v_off, b_voff));
-  HIP_TRY(hipMalloc(&u_off, b_uoff));
-  HIP_TRY(hipMalloc(&v_adj, b_adj));
-  HIP_TRY(hipMalloc(&u_adj, b_adj));
-  HIP_TRY(hipMalloc(&kUd, b_kU));
-  HIP_TRY(hipMalloc(&kVd, b_kV));
-  HIP_TRY(hipMemcpy(v_off, g.v_off.data(), b_voff, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(u_off, g.u_off.data(), b_uoff, hipMemcpyHostToDevice));
-  if (E) {
-    HIP_TRY(hipMemcpy(v_adj, g.v_adj.data(), (size_t)E * 4, hipMemcpyHostToDevice));
-    HIP_TRY(hipMemcpy(u_adj, g.u_adj.data(), (size_t)E * 4, hipMemcpyHostToDevice));
+  // one allocation for the six arrays, 256-byte aligned
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t b_voff = (size_t)(nV + 1) * 8, b_uoff = (size_t)(nU + 1) * 8;
+  const size_t b_adj = (size_t)E * 4, b_kU = (size_t)nU * 8, b_kV = (size_t)nV * 8;
+  const size_t o_uoff = up(b_voff), o_vadj = o_uoff + up(b_uoff), o_uadj = o_vadj + up(b_adj),
+               o_kU = o_uadj + up(b_adj), o_kV = o_kU + up(b_kU), total = o_kV + up(b_kV);
+  HIP_TRY(hipMalloc(&block, total));
+  v_off = (int64_t*)block;
+  u_off = (int64_t*)(block + o_uoff);
+  v_adj = (uint32_t*)(block + o_vadj);
+  u_adj = (uint32_t*)(block + o_uadj);
+  kUd = (uint64_t*)(block + o_kU);
+  kVd = (uint64_t*)(block + o_kV);
+  const struct { size_t at; const void* src; size_t bytes; } part[] = {
+      {0, g.v_off.data(), b_voff}, {o_uoff, g.u_off.data(), b_uoff},
+      {o_vadj, g.v_adj.data(), b_adj}, {o_uadj, g.u_adj.data(), b_adj},
+      {o_kU, kU.data(), b_kU}, {o_kV, kV.data(), b_kV}};
+  if (total <= (1u << 20)) {
+    // a small graph: one copy instead of six (each costs more than its bytes)
+    std::vector<char> host(total);
+    for (const auto& p : part)
+      if (p.bytes) memcpy(host.data() + p.at, p.src, p.bytes);
+    HIP_TRY(hipMemcpy(block, host.data(), total, hipMemcpyHostToDevice));
+  } else {
+    for (const auto& p : part)
+      if (p.bytes) HIP_TRY(hipMemcpy(block + p.at, p.src, p.bytes, hipMemcpyHostToDevice));
   }
-  if (nU) HIP_TRY(hipMemcpy(kUd, kU.data(), (size_t)nU * 8, hipMemcpyHostToDevice));
-  if (nV) HIP_TRY(hipMemcpy(kVd, kV.data(), (size_t)nV * 8, hipMemcpyHostToDevice));
   return GMBE_OK;
 }
 
 void DeviceGraph::release() {
-  (void)hipFree(v_off);
-  (void)hipFree(u_off);
-  (void)hipFree(v_adj);
-  (void)hipFree(u_adj);
-  (void)hipFree(kUd);
-  (void)hipFree(kVd);
+  (void)hipFree(block);
+  block = nullptr;
   v_off = u_off = nullptr;
   v_adj = u_adj = nullptr;
   kUd = kVd = nullptr;
@@ -282,7 +336,7 @@ struct gmbe_finder {
   int sel = 2, bound_height = 20, bound_size = 1500;
   // knobs
   int64_t waves_per_block = 4, blocks = 0, prune = 1, max_prefix = 4, lds_kb = 7;
-  int64_t queue_log2 = 22, list_cap = 0, arena_kb = 16384, root_stride = 1, root_phase = 0;
+  int64_t queue_log2 = -1, list_cap = 0, arena_kb = 16384, root_stride = 1, root_phase = 0;
   int64_t root_begin = 0, root_end = -1;  // processing-order rank range, -1 = all
   int64_t deadline_ms = 0;                 // 0 = run to completion
   int64_t late_share = 32;                 // 0 = off
@@ -309,7 +363,8 @@ struct gmbe_finder {
   // control counters, each on its own 256-byte line (kCtlStride u64 apart):
   // root_next, work_left, queued, list_cursor, n_deferred, then per-shard head/tail
   unsigned long long* ctl = nullptr;
-  unsigned long long* acc = nullptr;
+  unsigned long long* acc = nullptr;  // in ctl's allocation, with the graph table
+  unsigned long long* out = nullptr;  // pinned: the words of run_result
   uint32_t* list = nullptr;
   uint64_t list_words = 0;
   mbe::Task* deferred = nullptr;
@@ -317,7 +372,7 @@ struct gmbe_finder {
   int64_t exit_stamps = 0;              // knob: record per-block exit times
   unsigned long long* stamps = nullptr;  // 1 + nblocks: launch stamp, then per block
   std::vector<double> exit_s;            // per-block exit, seconds after launch
-  uint64_t deferred_cap = 1ull << 20;
+  uint64_t deferred_cap = 0;
   uint64_t last_deferred = 0;
   hipStream_t stream = nullptr;
   hipEvent_t ev0 = nullptr, ev1 = nullptr, evm = nullptr;  // evm: end of the main kernel
@@ -329,17 +384,45 @@ struct gmbe_finder {
 
 using namespace gmbe;
 
+// Control words run_result copies: the slots below C_QCTL.
+constexpr int kOutCtl = C_QCTL;
+
 static int finder_alloc(gmbe_finder* f) {
   KernelChoice kc = pick_kernel((int)f->lds_kb, (int)f->waves_per_block, false);
-  int blocks = f->blocks > 0 ? (int)f->blocks : resident_blocks(kc, f->eng.cu_count);
+  // unless set: as many waves as are resident at once, but no more than the
+  // graph can occupy -- one per top-level vertex, or one per 64 edges of the
+  // 2-hop passes where subtrees may be shared.  The 61 top-level vertices of a
+  // 400-edge graph ran 134 us on 4,096 waves, most of it waves that contend for
+  // the claim counter and sleep.
+  int blocks = (int)f->blocks;
+  if (blocks <= 0) {
+    const uint64_t want = std::max<uint64_t>(std::max<uint64_t>(f->dg.nV, f->dg.cost / 64), 1);
+    blocks = (int)std::min<uint64_t>((uint64_t)resident_blocks(kc, f->eng.cu_count),
+                                     (want + kc.waves - 1) / kc.waves);
+  }
   int nwaves = blocks * kc.waves;
-  // unless set, the list arena and the context slots are sized for the graph:
-  // a list holds at most |V| entries of <= 60 bytes
-  const uint64_t nv = f->dg.nV;
-  const int64_t arena_kb = f->arena_set ? f->arena_kb
-                                        : std::min<int64_t>(16384, std::max<int64_t>(4096, (int64_t)(nv * 24 * 64 / 1024)));
-  const int64_t ctx_kb = f->ctx_set ? f->ctx_kb
-                                    : std::min<int64_t>(1024, std::max<int64_t>(256, (int64_t)(nv * 16 / 1024)));
+  // unless set, the list arena and the context slots are sized for the graph.
+  // A list holds at most one entry per candidate (max_cand), and the lists of
+  // one path are at most one per vertex of L, so `need` covers every path, the
+  // re-indexed copy and a merge table; where that is less than the general
+  // size (4-16 MB by |V|) it is the whole arena: 34 GB of slabs for a graph of
+  // 12,000 edges took a second to give back.
+  const uint64_t nv = f->dg.nV, mc = f->dg.max_cand, d = f->dg.dmaxV;
+  uint64_t words = 1;
+  while (words < (uint64_t)mbe::kMaxW && words * 64 < d) words *= 2;
+  const uint64_t rec = 16 + 8 * words, levels = std::min<uint64_t>(d, 64 * mbe::kMaxW) + 4;
+  const uint64_t need = levels * mc * rec + mc * 24 + 4 * mc * 32 + 64 * 32 + 16 * d + 4096;
+  const uint64_t need_ctx = sizeof(mbe::CtxHdr) + mc * (rec + 4) + 8 * d + 1024;
+  auto kb = [](uint64_t bytes) { return (int64_t)((bytes + 1023) / 1024); };
+  int64_t arena_kb = f->arena_kb, ctx_kb = f->ctx_kb;
+  if (!f->arena_set) {
+    arena_kb = std::min<int64_t>(16384, std::max<int64_t>(4096, (int64_t)(nv * 24 * 64 / 1024)));
+    arena_kb = std::min(arena_kb, std::max<int64_t>(64, kb(need)));
+  }
+  if (!f->ctx_set) {
+    ctx_kb = std::min<int64_t>(1024, std::max<int64_t>(256, (int64_t)(nv * 16 / 1024)));
+    ctx_kb = std::min(ctx_kb, std::max<int64_t>(4, kb(need_ctx)));
+  }
   f->arena_kb = arena_kb;
   f->ctx_kb = ctx_kb;
   mbe::Scratch lay = scratch_layout(f->dg.nV, f->dg.dmaxV, (uint64_t)arena_kb * 1024ull,
@@ -353,14 +436,21 @@ static int finder_alloc(gmbe_finder* f) {
     if (e != hipSuccess)
       return set_error(GMBE_ERR_NOMEM, "scratch of %llu bytes (%d waves): %s",
                        (unsigned long long)bytes, nwaves, hipGetErrorString(e));
-    HIP_TRY(hipMemsetAsync(f->scratch, 0, bytes, f->stream));
     f->scratch_bytes = bytes;
+    lay.base = f->scratch;
+    HIP_TRY(launch_zero_slabs(f->stream, lay, (unsigned long long)nwaves));
   }
   lay.base = f->scratch;
   f->layout = lay;
   f->nwaves = nwaves;
   f->nblocks = blocks;
-  uint64_t qcap = (1ull << f->queue_log2) / kShards;  // slots per shard (a power of two)
+  // slots per shard (a power of two); unless set, room in one shard for four of
+  // the longest lists and in all for 16 entries a wave, at most 2^22 in total
+  uint64_t qcap = f->queue_log2 >= 0 ? (1ull << f->queue_log2) / kShards : 64;
+  if (f->queue_log2 < 0)
+    while (qcap < (1ull << 22) / kShards &&
+           (qcap * 15 < 4 * mc || qcap * kShards < 16ull * (uint64_t)nwaves))
+      qcap *= 2;
   // at least two: a slot's sequence number tells "holds position p" (p + 1)
   // from "free for position p + qcap" (p + qcap) only when qcap >= 2
   if (qcap < 2) qcap = 2;
@@ -373,7 +463,11 @@ static int finder_alloc(gmbe_finder* f) {
     HIP_TRY(hipMalloc(&f->qseq, qcap * kShards * 8));
     f->qcap = qcap;
   }
-  if (!f->deferred) HIP_TRY(hipMalloc(&f->deferred, f->deferred_cap * sizeof(mbe::Task)));
+  if (!f->deferred) {
+    // only a task whose L is wider than the main kernel's bitsets is deferred
+    f->deferred_cap = d > 64ull * mbe::kMainW ? 1ull << 20 : 64;
+    HIP_TRY(hipMalloc(&f->deferred, f->deferred_cap * sizeof(mbe::Task)));
+  }
   if ((uint64_t)f->list_cap != f->list_words) {
     if (f->list) (void)hipFree(f->list);
     f->list = nullptr;
@@ -413,13 +507,17 @@ static int gmbe_finder_create_impl(const gmbe_graph* g, int sel, int bound_heigh
     return set_error(GMBE_ERR_HIP, "stream/event creation failed");
   }
   rc = f->dg.upload(*g);
-  if (rc == GMBE_OK &&
-      hipMalloc(&f->ctl, C_NSLOTS * kCtlStride * sizeof(unsigned long long)) != hipSuccess)
+  // control block, result block and graph table in one allocation
+  const size_t b_ctl = kCtlWords * 8, b_acc = ((size_t)mbe::A_COUNT * 8 + 255) & ~(size_t)255;
+  if (rc == GMBE_OK && hipMalloc(&f->ctl, b_ctl + b_acc + sizeof(mbe::DevGraph)) != hipSuccess)
     rc = set_error(GMBE_ERR_NOMEM, "control block");
-  if (rc == GMBE_OK && hipMalloc(&f->acc, mbe::A_COUNT * sizeof(unsigned long long)) != hipSuccess)
-    rc = set_error(GMBE_ERR_NOMEM, "result block");
-  if (rc == GMBE_OK && hipMalloc(&f->gt, sizeof(mbe::DevGraph)) != hipSuccess)
-    rc = set_error(GMBE_ERR_NOMEM, "graph table");
+  if (rc == GMBE_OK && hipHostMalloc((void**)&f->out, (kOutCtl + mbe::A_COUNT) * 8,
+                                     hipHostMallocDefault) != hipSuccess)
+    rc = set_error(GMBE_ERR_NOMEM, "result words");
+  if (rc == GMBE_OK) {
+    f->acc = (unsigned long long*)((char*)f->ctl + b_ctl);
+    f->gt = (mbe::DevGraph*)((char*)f->acc + b_acc);
+  }
   if (rc) {
     gmbe_finder_destroy(f);
     return rc;
@@ -509,22 +607,11 @@ static int gmbe_finder_execute_impl(gmbe_finder* f, gmbe_result* res) {
   const uint64_t b = (uint64_t)f->root_begin;
   const uint64_t first = b + ((uint64_t)f->root_phase + stride - b % stride) % stride;
   const uint64_t n_roots = end > first ? (end - first + stride - 1) / stride : 0;
-  std::vector<unsigned long long> ctl_h(C_NSLOTS * kCtlStride, 0ull);
-  ctl_h[C_WORK_LEFT * kCtlStride] = n_roots;
-  HIP_TRY(hipMemcpyAsync(f->ctl, ctl_h.data(), ctl_h.size() * 8, hipMemcpyHostToDevice,
-                         f->stream));
-  HIP_TRY(hipMemsetAsync(f->acc, 0, mbe::A_COUNT * 8, f->stream));
-  hipLaunchKernelGGL(mbe::init_queue, dim3(256), dim3(256), 0, f->stream, f->qseq,
-                     (unsigned long long)f->qcap);
-  HIP_TRY(hipGetLastError());
   mbe::Params P{};
-  {
-    // the graph table of a finder: one entry
-    mbe::DevGraph e = f->dg.view();
-    e.bound_height = f->bound_height;
-    e.bound_size = f->bound_size;
-    HIP_TRY(hipMemcpyAsync(f->gt, &e, sizeof(e), hipMemcpyHostToDevice, f->stream));
-  }
+  // the graph table of a finder: one entry
+  mbe::DevGraph entry = f->dg.view();
+  entry.bound_height = f->bound_height;
+  entry.bound_size = f->bound_size;
   P.gt = f->gt;
   P.per_graph = nullptr;
   P.s.root_next = f->ctl + C_ROOT_NEXT * kCtlStride;
@@ -573,8 +660,13 @@ static int gmbe_finder_execute_impl(gmbe_finder* f, gmbe_result* res) {
   P.share_work = (int)std::min<int64_t>(f->share_work, INT32_MAX);
   P.share_queue = f->share_queue >= 0 ? (int)f->share_queue : f->nwaves;
   KernelChoice kc = pick_kernel((int)f->lds_kb, (int)f->waves_per_block, false);
-  hipLaunchKernelGGL(mbe::reset_ctx, dim3(64), dim3(256), 0, f->stream, P,
-                     (unsigned long long)f->nwaves * (unsigned long long)f->ctx_slots);
+  const unsigned long long n_ctx = (unsigned long long)f->nwaves * (unsigned long long)f->ctx_slots;
+  const unsigned long long most = std::max<unsigned long long>(
+      std::max<unsigned long long>(kCtlWords, f->qcap * kShards), n_ctx);
+  hipLaunchKernelGGL(mbe::run_start, dim3((unsigned)std::min<unsigned long long>((most + 255) / 256, 512)),
+                     dim3(256), 0, f->stream, P, f->ctl, (unsigned long long)kCtlWords,
+                     (unsigned long long)C_WORK_LEFT * kCtlStride, (unsigned long long)n_roots,
+                     n_ctx, f->gt, entry);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipEventRecord(f->ev0, f->stream));
   if (n_roots > 0) {
@@ -582,24 +674,28 @@ static int gmbe_finder_execute_impl(gmbe_finder* f, gmbe_result* res) {
     HIP_TRY(hipGetLastError());
   }
   HIP_TRY(hipEventRecord(f->evm, f->stream));
-  std::vector<unsigned long long> ctl_out(C_NSLOTS * kCtlStride, 0ull);
-  HIP_TRY(hipMemcpyAsync(ctl_out.data(), f->ctl, ctl_out.size() * 8, hipMemcpyDeviceToHost,
-                         f->stream));
-  HIP_TRY(hipMemcpyAsync(f->main_acc, f->acc, sizeof(f->main_acc), hipMemcpyDeviceToHost,
-                         f->stream));
-  HIP_TRY(hipStreamSynchronize(f->stream));
-  f->last_deferred = std::min<uint64_t>(ctl_out[C_DEFERRED * kCtlStride], f->deferred_cap);
+  // what the host needs of a pass: f->out[slot] of the control block, then the counters
+  auto fetch = [&]() -> hipError_t {
+    hipLaunchKernelGGL(mbe::run_result, dim3(1), dim3(128), 0, f->stream, f->ctl,
+                       (unsigned long long)kCtlStride, kOutCtl, f->acc, f->out);
+    hipError_t e = hipGetLastError();
+    return e != hipSuccess ? e : hipStreamSynchronize(f->stream);
+  };
+  HIP_TRY(fetch());
+  memcpy(f->main_acc, f->out + kOutCtl, sizeof(f->main_acc));
+  f->last_deferred = std::min<uint64_t>(f->out[C_DEFERRED], f->deferred_cap);
   // the wide pass gets what is left of the budget
   const double used_ms = (now_s() - t0) * 1e3;
   const bool out_of_time = f->deadline_ms > 0 && used_ms >= (double)f->deadline_ms;
   if (f->deadline_ms > 0 && !out_of_time)
     P.budget = (uint64_t)(((double)f->deadline_ms - used_ms) * f->eng.wall_khz);
+  bool wide = false;
   if (f->last_deferred > 0 && !out_of_time) {
     // wide-bitset pass over the deferred tasks (same queue, fresh counters)
     std::vector<unsigned long long> ctl2(C_NSLOTS * kCtlStride, 0ull);
     ctl2[C_WORK_LEFT * kCtlStride] = f->last_deferred;
-    ctl2[C_LIST_CURSOR * kCtlStride] = ctl_out[C_LIST_CURSOR * kCtlStride];
-    ctl2[C_DEADLINE * kCtlStride] = ctl_out[C_DEADLINE * kCtlStride];
+    ctl2[C_LIST_CURSOR * kCtlStride] = f->out[C_LIST_CURSOR];
+    ctl2[C_DEADLINE * kCtlStride] = f->out[C_DEADLINE];
     HIP_TRY(hipMemcpyAsync(f->ctl, ctl2.data(), ctl2.size() * 8, hipMemcpyHostToDevice,
                            f->stream));
     hipLaunchKernelGGL(mbe::init_queue, dim3(256), dim3(256), 0, f->stream, f->qseq,
@@ -617,19 +713,19 @@ static int gmbe_finder_execute_impl(gmbe_finder* f, gmbe_result* res) {
                             : f->nblocks;
     hipLaunchKernelGGL(wk.fn, dim3(wblocks), dim3(wk.waves * 64), 0, f->stream, P);
     HIP_TRY(hipGetLastError());
+    HIP_TRY(hipEventRecord(f->ev1, f->stream));
+    HIP_TRY(fetch());
+    wide = true;
   }
-  HIP_TRY(hipEventRecord(f->ev1, f->stream));
-  unsigned long long acc_h[mbe::A_COUNT];
-  HIP_TRY(hipMemcpyAsync(acc_h, f->acc, sizeof(acc_h), hipMemcpyDeviceToHost, f->stream));
-  HIP_TRY(hipMemcpyAsync(ctl_out.data(), f->ctl, ctl_out.size() * 8, hipMemcpyDeviceToHost,
-                         f->stream));
-  HIP_TRY(hipStreamSynchronize(f->stream));
+  const unsigned long long* acc_h = f->out + kOutCtl;
+  const uint64_t work_left = f->out[C_WORK_LEFT];
   double t1 = now_s();
   float ms = 0, mms = 0;
-  HIP_TRY(hipEventElapsedTime(&ms, f->ev0, f->ev1));
   HIP_TRY(hipEventElapsedTime(&mms, f->ev0, f->evm));
+  ms = mms;
+  if (wide) HIP_TRY(hipEventElapsedTime(&ms, f->ev0, f->ev1));
   f->main_ms = mms;
-  f->wide_ms = f->last_deferred > 0 ? (double)ms - mms : 0.0;
+  f->wide_ms = wide ? (double)ms - mms : 0.0;
   res->maximal = acc_h[mbe::A_MAXIMAL];
   res->non_maximal = acc_h[mbe::A_NONMAX];
   res->hash_sum = acc_h[mbe::A_HSUM];
@@ -642,9 +738,9 @@ static int gmbe_finder_execute_impl(gmbe_finder* f, gmbe_result* res) {
   res->exe_time_s = t1 - t0;
   res->kernel_time_s = ms * 1e-3;
   f->ran = true;
-  f->list_used = std::min<uint64_t>(ctl_out[C_LIST_CURSOR * kCtlStride], f->list_words);
+  f->list_used = std::min<uint64_t>(f->out[C_LIST_CURSOR], f->list_words);
   f->list_ovf = acc_h[mbe::A_LIST_OVF];
-  memcpy(f->prof, acc_h, sizeof(acc_h));
+  memcpy(f->prof, acc_h, sizeof(f->prof));
   f->exit_s.clear();
   if (P.exit_stamps && n_roots > 0) {
     std::vector<unsigned long long> st(2ull * f->nblocks);
@@ -654,9 +750,9 @@ static int gmbe_finder_execute_impl(gmbe_finder* f, gmbe_result* res) {
     for (int b = 0; b < f->nblocks; ++b)
       f->exit_s.push_back((double)(st[2 * b + 1] - t0s) / ((double)f->eng.wall_khz * 1e3));
   }
-  const uint64_t roots_claimed = std::min<uint64_t>(ctl_out[C_ROOT_NEXT * kCtlStride], n_roots);
+  const uint64_t roots_claimed = std::min<uint64_t>(f->out[C_ROOT_NEXT], n_roots);
   if (f->deadline_ms > 0 &&
-      (acc_h[mbe::A_ABANDONED] > 0 || ctl_out[C_WORK_LEFT * kCtlStride] != 0 ||
+      (acc_h[mbe::A_ABANDONED] > 0 || work_left != 0 ||
        (f->last_deferred > 0 && out_of_time)))
     return set_error(GMBE_ERR_DEADLINE,
                      "deadline of %lld ms passed: %llu of %llu top-level vertices claimed, %llu "
@@ -765,8 +861,7 @@ void gmbe_finder_destroy(gmbe_finder* f) {
   (void)hipFree(f->q);
   (void)hipFree(f->qseq);
   (void)hipFree(f->ctl);
-  (void)hipFree(f->acc);
-  (void)hipFree(f->gt);
+  if (f->out) (void)hipHostFree(f->out);
   (void)hipFree(f->stamps);
   (void)hipFree(f->list);
   (void)hipFree(f->deferred);

@@ -221,9 +221,10 @@ int Lane::alloc_run() {
       return set_error(GMBE_ERR_NOMEM, "lane scratch of %llu bytes (%d waves): %s",
                        (unsigned long long)bytes, nw, hipGetErrorString(e));
     scratch_bytes = bytes;
-    // slabs start zeroed (the candidate maps rely on it); a kernel, not a
+    // the count maps and bitmaps of the slabs start zeroed; a kernel, not a
     // memset, so that nothing here differs between eager and captured use
-    LANE_TRY(launch_fill(st, (unsigned long long*)scratch, bytes / 8, 0ull));
+    lay.base = scratch;
+    LANE_TRY(launch_zero_slabs(st, lay, (unsigned long long)nw));
   }
   lay.base = scratch;
   layout = lay;

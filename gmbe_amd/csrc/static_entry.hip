@@ -10,6 +10,7 @@
 #include <algorithm>
 #include <cstring>
 #include <mutex>
+#include <vector>
 
 #include "device_graph.hpp"
 #include "graph.hpp"
@@ -109,8 +110,9 @@ static int execute_static_impl(const gmbe_graph* g, int bound_height, int bound_
   };
   const uint64_t o_voff = take((nV + 1) * 8), o_uoff = take((nU + 1) * 8);
   const uint64_t o_vadj = take(E * 4), o_uadj = take(E * 4);
-  const uint64_t o_kU = take(nU * 8), o_kV = take(nV * 8);
   const uint64_t o_uorig = take(nU * 4), o_vorig = take(nV * 4);
+  const uint64_t b_graph = o;  // what the host copies in
+  const uint64_t o_kU = take(nU * 8), o_kV = take(nV * 8);
   const uint64_t o_gt = take(sizeof(mbe::DevGraph));
   const uint64_t o_ctl = take(kCtlWords * 8), o_acc = take(mbe::A_COUNT * 8);
   const uint64_t o_q = take(kStaticQcap * mbe::kShards * mbe::kEntryWords * 4);
@@ -138,14 +140,20 @@ static int execute_static_impl(const gmbe_graph* g, int bound_height, int bound_
   hipStream_t st = nullptr;  // the null stream: no stream is created
   const double t0 = now_s();
   // the graph (host -> the array), its keys computed on the device
-  S_TRY(hipMemcpy(base + o_voff, g->v_off.data(), (nV + 1) * 8, hipMemcpyHostToDevice));
-  S_TRY(hipMemcpy(base + o_uoff, g->u_off.data(), (nU + 1) * 8, hipMemcpyHostToDevice));
-  if (E) {
-    S_TRY(hipMemcpy(base + o_vadj, g->v_adj.data(), E * 4, hipMemcpyHostToDevice));
-    S_TRY(hipMemcpy(base + o_uadj, g->u_adj.data(), E * 4, hipMemcpyHostToDevice));
+  const struct { uint64_t at; const void* src; uint64_t bytes; } part[] = {
+      {o_voff, g->v_off.data(), (nV + 1) * 8}, {o_uoff, g->u_off.data(), (nU + 1) * 8},
+      {o_vadj, g->v_adj.data(), E * 4}, {o_uadj, g->u_adj.data(), E * 4},
+      {o_uorig, g->u_orig.data(), nU * 4}, {o_vorig, g->v_orig.data(), nV * 4}};
+  if (b_graph <= (1u << 20)) {
+    // a small graph: one copy instead of six (each costs more than its bytes)
+    std::vector<char> host(b_graph);
+    for (const auto& p : part)
+      if (p.bytes) memcpy(host.data() + p.at, p.src, p.bytes);
+    S_TRY(hipMemcpy(base, host.data(), b_graph, hipMemcpyHostToDevice));
+  } else {
+    for (const auto& p : part)
+      if (p.bytes) S_TRY(hipMemcpy(base + p.at, p.src, p.bytes, hipMemcpyHostToDevice));
   }
-  if (nU) S_TRY(hipMemcpy(base + o_uorig, g->u_orig.data(), nU * 4, hipMemcpyHostToDevice));
-  if (nV) S_TRY(hipMemcpy(base + o_vorig, g->v_orig.data(), nV * 4, hipMemcpyHostToDevice));
   const uint32_t sideU = g->swapped ? 1 : 0, sideV = g->swapped ? 0 : 1;
   if (nU)
     hipLaunchKernelGGL(mbe::static_keys, dim3(64), dim3(256), 0, st, (uint64_t*)(base + o_kU),
@@ -175,7 +183,7 @@ static int execute_static_impl(const gmbe_graph* g, int bound_height, int bound_
   unsigned long long* ctl = (unsigned long long*)(base + o_ctl);
   unsigned long long* acc = (unsigned long long*)(base + o_acc);
   unsigned long long* qseq = (unsigned long long*)(base + o_qseq);
-  S_TRY(launch_fill(st, (unsigned long long*)lay.base, nwaves * lay.slab / 8, 0ull));
+  S_TRY(launch_zero_slabs(st, lay, nwaves));
   S_TRY(launch_fill(st, acc, mbe::A_COUNT, 0ull));
   S_TRY(launch_ctl_start(st, ctl, nV));
   S_TRY(launch_init_queue(st, qseq, kStaticQcap));

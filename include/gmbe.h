@@ -186,12 +186,14 @@ int gmbe_finder_create(const gmbe_graph* g, int sel, int bound_height,
 /* Tuning knobs, set before execute (the reference's compile-time macros,
  * src/CMakeLists.txt:13-39, src/GpuUtil.cuh:9-24, src/IterFinderGpu.cu:912-917):
  *   "waves_per_block" (2, 4 or 8), "blocks", "queue_log2" (0..30: 2^queue_log2
- *   queue entries over 32 shards, at least two per shard), "list_cap" (u32
+ *   queue entries over 32 shards, at least two per shard; unless set, sized
+ *   for the graph and the waves), "list_cap" (u32
  *   words of list output; 0 = off), "prune" (0/1, PRUNE_EN), "max_prefix"
  *   (2..8), "bound_height", "bound_size".
  * Scheduler and memory knobs (no counterpart): "lds_kb" (LDS list arena per
  *   wave: 0, 3, 7 or 16; default 7), "arena_kb" and "ctx_kb" (per wave;
- *   unless set they scale with |V|: 4-16 MB and 256 KB-1 MB), "ctx_slots",
+ *   unless set what the graph's lists can fill at most, within 4-16 MB and
+ *   256 KB-1 MB scaled with |V|), "ctx_slots",
  *   "group", "share", "share_work", "share_queue", "merge_min",
  *   "merge_branch", "late_share", "profile", "dom_k" (0..16 dominators per
  *   list reduction; 0 = off), "dom_skip" (0/1: mark pushes inside a
