@@ -310,14 +310,12 @@ mbe::Scratch scratch_layout(uint32_t nV, uint32_t dmaxV, uint64_t arena_bytes,
   s.o_T = take(d * 4);
   s.o_kL = take(d * 8);
   s.o_U = take(nv * 4);
-  s.o_Ucnt = take(nv * 4);
   s.o_C = take(nv * 4);
-  s.o_kC = take(nv * 8);
   s.o_R = take(nv * 4);
   s.o_fr = take((d + 2) * sizeof(mbe::Frame));
   // small_dfs saves its stack over the arrays of the task's root phase, which
   // are dead by then, where they are large enough
-  s.o_save = nv * 24 >= (uint64_t)mbe::kSaveWords * 4 ? s.o_U : take((uint64_t)mbe::kSaveWords * 4);
+  s.o_save = nv * 12 >= (uint64_t)mbe::kSaveWords * 4 ? s.o_U : take((uint64_t)mbe::kSaveWords * 4);
   s.o_arena = take(arena_bytes);
   s.arena_bytes = arena_bytes;
   s.o_ctx = take(ctx_bytes * ctx_slots);

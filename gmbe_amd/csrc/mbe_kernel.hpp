@@ -117,7 +117,7 @@ struct Scratch {
   char* base;        // per-wave slabs
   uint64_t slab;     // bytes per wave
   // offsets inside a slab
-  uint64_t o_cmap, o_bm0, o_bm1, o_L, o_Lp, o_T, o_kL, o_U, o_Ucnt, o_C, o_kC, o_R, o_fr,
+  uint64_t o_cmap, o_bm0, o_bm1, o_L, o_Lp, o_T, o_kL, o_U, o_C, o_R, o_fr,
       o_save, o_arena, o_ctx;
   uint64_t arena_bytes, ctx_bytes;  // ctx_bytes: per context slot
   uint32_t ctx_slots;                // context slots per wave
@@ -201,6 +201,16 @@ constexpr int kCounters = (int)(sizeof(Counters) / sizeof(LdsCount));
 #include "small_dfs.hpp"
 
 namespace mbe {
+
+// The launch's Params for a leaf function: the kernel's argument segment, read
+// with scalar loads.
+typedef const __attribute__((address_space(4))) Params* ParamsPtr;
+__device__ __forceinline__ uint64_t kernel_params() {
+  return (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+}
+__device__ __forceinline__ const Params& leaf_params(uint64_t kp) {
+  return *(const Params*)(ParamsPtr)uni64(kp);
+}
 
 // Per-graph result counters of a batch (u64 each, kPerGraph per graph).
 enum PerGraph : int {
@@ -324,14 +334,21 @@ __device__ __forceinline__ uint32_t wave_intersect_count(const uint32_t* A, uint
   return cnt;
 }
 
-// f(j, w) for every edge (L[j], w), w in N(L[j]) over the U->V rows.  The
-// edges of 64 L vertices at a time are flattened across lanes; each lane
-// finds its vertex by binary search over the 64 prefix offsets kept in LDS.
+// f(j, w, ok) for the edges (L[j], w), w in N(L[j]) over the U->V rows, kEdges
+// per lane at a time (ok marks the ones that exist).  The edges of 64 L
+// vertices are flattened across lanes; each lane finds its vertex by binary
+// search over the 64 prefix offsets kept in LDS (six fixed steps: offsets past
+// the last vertex equal the total, which no edge reaches).  A wave alone on a
+// SIMD hides no latency but its own: with one edge per lane in flight a hub's
+// 30,000-edge pass took 2.5 us per 64 edges.
+constexpr int kEdges = 4;
 template <class F>
 __device__ __forceinline__ uint64_t for_each_edge(const uint32_t* L, uint32_t nL, const int64_t* off,
                                   const uint32_t* adj, uint32_t* s_off, int64_t* s_start, F&& f) {
   uint32_t lane = lane_id();
   uint64_t edges = 0;
+  auto* lo_off = as_lds(s_off);
+  auto* lo_start = as_lds(s_start);
   for (uint32_t base = 0; base < nL; base += kWave) {
     uint32_t j = base + lane;
     uint32_t deg = 0;
@@ -343,21 +360,33 @@ __device__ __forceinline__ uint64_t for_each_edge(const uint32_t* L, uint32_t nL
     }
     uint32_t incl = wave_incl_scan32(deg);
     uint32_t total = read_lane(incl, kWave - 1);
-    uint32_t nb = nL - base < (uint32_t)kWave ? nL - base : (uint32_t)kWave;
     edges += total;
-    s_off[lane] = incl - deg;
-    s_start[lane] = st;
-    wave_sync();
-    for (uint32_t t = lane; t < total; t += kWave) {
-      uint32_t lo = 0, hi = nb - 1;
-      while (lo < hi) {
-        uint32_t mid = (lo + hi + 1) >> 1;
-        if (s_off[mid] <= t) lo = mid; else hi = mid - 1;
+    lo_off[lane] = incl - deg;
+    lo_start[lane] = st - (int64_t)(incl - deg);
+    wave_mem_wait();
+    for (uint32_t t0 = 0; t0 < total; t0 += kEdges * kWave) {
+      uint32_t at[kEdges], w[kEdges];
+      bool ok[kEdges];
+#pragma unroll
+      for (int e = 0; e < kEdges; ++e) at[e] = 0;
+#pragma unroll
+      for (uint32_t step = 32; step > 0; step >>= 1) {
+#pragma unroll
+        for (int e = 0; e < kEdges; ++e) {
+          const uint32_t t = t0 + e * kWave + lane;
+          if (lo_off[at[e] + step] <= t) at[e] += step;
+        }
       }
-      int64_t e = s_start[lo] + (int64_t)(t - s_off[lo]);
-      f(base + lo, adj[e]);
+#pragma unroll
+      for (int e = 0; e < kEdges; ++e) {
+        const uint32_t t = t0 + e * kWave + lane;
+        ok[e] = t < total;
+        w[e] = ok[e] ? adj[lo_start[at[e]] + (int64_t)t] : 0;
+        at[e] += base;
+      }
+      f(at, w, ok);
     }
-    wave_sync();
+    wave_mem_wait();
   }
   return edges;
 }
@@ -375,9 +404,13 @@ __device__ __forceinline__ uint64_t for_each_edge(const uint32_t* L, uint32_t nL
 constexpr int kChunk = 24;      // children per entry
 constexpr int kEntryWords = 32; // hdr, prefix[7], children[24]
 
+// Longest nap of a wave without work, in units of 2,048 cycles.  A run ends, and
+// a shared subtree starts, one nap late at worst; shorter naps poll more often.
+constexpr uint32_t kMaxNap = 8;
+
 __device__ __forceinline__ void backoff(uint32_t& n) {
   for (uint32_t i = 0; i < n; ++i) __builtin_amdgcn_s_sleep(32);
-  n = n < 64 ? n * 2 : 64;
+  n = n < kMaxNap ? n * 2 : kMaxNap;
 }
 
 __device__ __forceinline__ unsigned long long* shard_head(const Sched& s, uint32_t sh) {
@@ -576,9 +609,7 @@ struct WaveMem {
   uint32_t* T;     // temporary
   uint64_t* kL;    // hash keys of L
   uint32_t* U;     // 2-hop set, ascending
-  uint32_t* Ucnt;  // |N(w) ∩ L|
   uint32_t* C;     // candidates
-  uint64_t* kC;    // hash keys of C
   uint32_t* R;     // closure of L
   Frame* fr;       // DFS frames (slab; the first kLdsFrames live in fr_lds)
   Frame* fr_lds;   // DFS frames in LDS
@@ -661,9 +692,7 @@ __device__ __forceinline__ WaveMem wave_mem(const Params& P, uint64_t gw, char* 
   m.T = (uint32_t*)(b + S.o_T);
   m.kL = (uint64_t*)(b + S.o_kL);
   m.U = (uint32_t*)(b + S.o_U);
-  m.Ucnt = (uint32_t*)(b + S.o_Ucnt);
   m.C = (uint32_t*)(b + S.o_C);
-  m.kC = (uint64_t*)(b + S.o_kC);
   m.R = (uint32_t*)(b + S.o_R);
   m.fr = (Frame*)(b + S.o_fr);
   m.fr_lds = fr_lds;
@@ -796,7 +825,7 @@ __device__ __forceinline__ T rd(const T* p) {
 
 struct PassOut {
   uint32_t cbranch;     // pushable entries of the child list
-  bool nonmax;
+  uint32_t nonmax;
   uint64_t absorbed;    // key sum of the groups joining R'
   uint64_t best_next;   // (rep << 32 | position) of the next push in the parent
   uint64_t best_child;  // same, for the child's first push
@@ -812,10 +841,20 @@ struct PassOut {
 // first of the child, are the first qualifying positions (a ballot per
 // chunk); otherwise they are minimum reps over the wave.
 // LDS_IN / LDS_OUT: the parent / child list is in LDS (ds_ accesses).
-template <int W, bool LIST_REMOTE, bool LDS_IN = false, bool LDS_OUT = false>
-__device__ __forceinline__ PassOut push_pass(Rec<W>* recs, uint32_t len, const uint64_t* ax, uint32_t xidx,
-                             Rec<W>* crec, bool prune, bool ordered) {
+// axv: lane w holds word w of ax.  flags: 1 prune, 2 ordered.
+template <int W, bool LIST_REMOTE, bool LDS_IN, bool LDS_OUT>
+MBE_LEAF PassOut push_leaf(Rec<W>* recs_, uint32_t len_, uint64_t axv, uint32_t xidx_, Rec<W>* crec_,
+                           uint32_t flags_) {
   const uint32_t lane = lane_id();
+  const uint32_t len = uni(len_), xidx = uni(xidx_), flags = uni(flags_);
+  const bool prune = flags & 1u, ordered = flags & 2u;
+  uint64_t ax[W];
+#pragma unroll
+  for (int w = 0; w < W; ++w) ax[w] = read_lane64(axv, w);
+  // one-word lists outside the LDS are in device memory; wider ones are
+  // reached through generic pointers wherever they are
+  auto* recs = uni_ptr(recs_);
+  auto* crec = uni_ptr(crec_);
   bool nonmax = false;
   // once the node is known to be non-maximal its child list is never used:
   // stop writing it (the prune marks and the next push still need every entry)
@@ -939,11 +978,29 @@ __device__ __forceinline__ PassOut push_pass(Rec<W>* recs, uint32_t len, const u
   }
   PassOut o;
   o.cbranch = cbranch;
-  o.nonmax = dead;
+  o.nonmax = dead ? 1u : 0u;
   o.absorbed = absorbed;
   o.best_next = ordered ? best_next : wave_min_pair(best_next);
   o.best_child = ordered ? best_child : wave_min_pair(best_child);
   o.clen = clen;
+  return o;
+}
+
+template <int W, bool LIST_REMOTE, bool LDS_IN = false, bool LDS_OUT = false>
+__device__ __forceinline__ PassOut push_pass(Rec<W>* recs, uint32_t len, const uint64_t* ax,
+                                             uint32_t xidx, Rec<W>* crec, bool prune,
+                                             bool ordered) {
+  uint64_t axv = 0;
+#pragma unroll
+  for (int w = 0; w < W; ++w) axv = write_lane64(axv, ax[w], w);
+  PassOut o = push_leaf<W, LIST_REMOTE, LDS_IN, LDS_OUT>(recs, len, axv, xidx, crec,
+                                                         (prune ? 1u : 0u) | (ordered ? 2u : 0u));
+  o.cbranch = uni(o.cbranch);
+  o.nonmax = uni(o.nonmax);
+  o.absorbed = uni64(o.absorbed);
+  o.best_next = uni64(o.best_next);
+  o.best_child = uni64(o.best_child);
+  o.clen = uni(o.clen);
   return o;
 }
 
@@ -1051,11 +1108,17 @@ constexpr int kItemsPerEntry = 15;  // (position, candidate) pairs after hdr, ow
 // (nothing published) when the queue lacks room or fewer than min_items
 // entries are left to push.
 template <int W, bool KL_R, bool C_R>
-__device__ __forceinline__ bool publish_list(const Params& P, uint64_t gw, uint32_t ctx, uint32_t gid,
-                             const Rec<W>* root, uint32_t len,
-                             uint32_t nL, uint32_t nC, uint32_t nbits, uint64_t sumR0,
-                             const TaskArrays& src, uint32_t min_rep = 0,
-                             uint32_t min_items = 1) {
+MBE_LEAF bool publish_leaf(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t gid_,
+                           const Rec<W>* root_, uint32_t len_, uint32_t nL_, uint32_t nC_,
+                           uint32_t nbits_, uint64_t sumR0_, const uint64_t* kL_,
+                           const uint32_t* C_, uint32_t min_rep_, uint32_t min_items_) {
+  const Params& P = leaf_params(kp);
+  const uint32_t gw = uni(gw_), ctx = uni(ctx_), gid = uni(gid_), len = uni(len_), nL = uni(nL_),
+                 nC = uni(nC_), nbits = uni(nbits_), min_rep = uni(min_rep_),
+                 min_items = uni(min_items_);
+  const uint64_t sumR0 = uni64(sumR0_);
+  const Rec<W>* root = uni_ptr(root_);
+  const TaskArrays src{uni_ptr(kL_), uni_ptr(C_)};
   const uint32_t lane = lane_id();
   const Sched& s = P.s;
   CtxHdr* h = ctx_hdr(P, ctx);
@@ -1154,14 +1217,28 @@ __device__ __forceinline__ bool publish_list(const Params& P, uint64_t gw, uint3
   return true;
 }
 
+template <int W, bool KL_R, bool C_R>
+__device__ __forceinline__ bool publish_list(const Params& P, uint64_t gw, uint32_t ctx,
+                                             uint32_t gid, const Rec<W>* root, uint32_t len,
+                                             uint32_t nL, uint32_t nC, uint32_t nbits,
+                                             uint64_t sumR0, const TaskArrays& src,
+                                             uint32_t min_rep = 0, uint32_t min_items = 1) {
+  return uni((uint32_t)publish_leaf<W, KL_R, C_R>(kernel_params(), (uint32_t)gw, ctx, gid, root,
+                                                  len, nL, nC, nbits, sumR0, src.kL, src.C,
+                                                  min_rep, min_items)) != 0;
+}
+
 // Publish a node of small_dfs (at most 64 entries, one per lane) as this wave's
 // context and push one item per entry still to be pushed: publish_list for a
 // list in registers.  Entries are renumbered by position, which keeps their
 // order, all that a push looks at.
-__device__ __forceinline__ bool publish_small(const Params& P, uint64_t gw, uint32_t ctx,
-                                              uint32_t gid, uint32_t nL, uint64_t a0, uint64_t ks,
-                                              uint64_t key, uint64_t L, uint64_t alive,
-                                              uint64_t push, uint64_t todo, uint64_t sumR) {
+MBE_LEAF bool publish_small(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t gid_, uint32_t nL_,
+                            uint64_t a0, uint64_t ks, uint64_t key,
+                            const __attribute__((address_space(3))) SmallCall* sc) {
+  const Params& P = leaf_params(kp);
+  const uint32_t gw = uni(gw_), ctx = uni(ctx_), gid = uni(gid_), nL = uni(nL_);
+  const uint64_t L = uni64(sc->sh_L), alive = uni64(sc->sh_alive), push = uni64(sc->sh_push),
+                 todo = uni64(sc->sh_todo), sumR = uni64(sc->sh_sumR);
   const uint32_t lane = lane_id();
   const Sched& s = P.s;
   const uint32_t len = (uint32_t)__popcll(alive), n_items = (uint32_t)__popcll(todo);
@@ -1258,9 +1335,8 @@ __device__ __forceinline__ void run_small(const Params& P, const WaveMem& m, uin
     }
     how = SMALL_RESUME;
     const uint32_t cx = free_ctx(P, gw);
-    if (cx != kNone &&
-        publish_small(P, gw, cx, gid, nL, a0, ks, key, uni64(sc->sh_L), uni64(sc->sh_alive),
-                      uni64(sc->sh_push), uni64(sc->sh_todo), uni64(sc->sh_sumR))) {
+    if (cx != kNone && uni((uint32_t)publish_small(kernel_params(), (uint32_t)gw, cx, gid, nL, a0,
+                                                   ks, key, sc))) {
       how = SMALL_RESUME_SHARED;
       ctr.splits++;
       ctr.publishes++;
@@ -1309,26 +1385,29 @@ __device__ __forceinline__ void run_small_list(const Params& P, const WaveMem& m
 // entry.  Returns the new length and recomputes the first push and the
 // pushable count; leaves the list unchanged (returns len) when the arenas
 // lack room for the table.
+struct MergeSlot {
+  unsigned long long id;  // hash << 32 | (first-inserted entry + 1); 0 = empty
+  uint32_t mi, rep;
+  uint64_t ksum;
+  uint32_t first;         // smallest entry of the slot
+  uint32_t pad;
+};
+// Length, first push (rep << 32 | position) and pushable count of a list.
+struct ListOut {
+  uint64_t best;
+  uint32_t len, cbranch;
+  uint32_t dropped, skipped;
+};
+
 template <int W>
-__device__ __forceinline__ uint32_t merge_twins_impl(const WaveMem& m, Rec<W>* crec, uint32_t len,
-                                                     uint32_t& lds_top, uint64_t& hbm_top,
-                                                     uint64_t& best_child, uint32_t& cbranch,
-                                                     bool ordered) {
+MBE_LEAF ListOut merge_leaf(Rec<W>* crec_, uint32_t len_, MergeSlot* tab_, uint32_t T_,
+                            uint32_t ordered_) {
   const uint32_t lane = lane_id();
-  struct Slot {
-    unsigned long long id;  // hash << 32 | (first-inserted entry + 1); 0 = empty
-    uint32_t mi, rep;
-    uint64_t ksum;
-    uint32_t first;         // smallest entry of the slot
-    uint32_t pad;
-  };
-  uint32_t T = 64;
-  while (T < 2 * len) T <<= 1;
-  uint32_t tier = 1;
-  uint64_t tb = 0;
-  const uint64_t taddr = arena_take(m, lds_top, hbm_top, (uint64_t)T * sizeof(Slot), tier, tb);
-  if (taddr == 0) return len;
-  Slot* tab = (Slot*)taddr;
+  const uint32_t len = uni(len_), T = uni(T_);
+  const bool ordered = uni(ordered_) != 0;
+  Rec<W>* crec = uni_ptr(crec_);
+  MergeSlot* tab = uni_ptr(tab_);
+  lds_flat_fence();
   for (uint32_t i = lane; i < T; i += kWave) {
     tab[i].id = 0;
     tab[i].mi = kNone;
@@ -1337,14 +1416,17 @@ __device__ __forceinline__ uint32_t merge_twins_impl(const WaveMem& m, Rec<W>* c
     tab[i].first = kNone;
   }
   wave_mem_wait();
+  // the next entry of a lane is loaded while this one's slot is found (an
+  // insertion writes only its own entry's minidx)
+  Rec<W> nx;
+  if (lane < len) nx = crec[lane];
   for (uint32_t i = lane; i < len; i += kWave) {
-    uint64_t key[W];
+    const Rec<W> me_ = nx;
+    if (i + kWave < len) nx = crec[i + kWave];
+    const uint64_t* key = me_.a;
     uint64_t hk = 0x2545F4914F6CDD1Dull;
 #pragma unroll
-    for (int w = 0; w < W; ++w) {
-      key[w] = crec[i].a[w];
-      hk = mix64(hk ^ key[w]);
-    }
+    for (int w = 0; w < W; ++w) hk = mix64(hk ^ key[w]);
     const unsigned long long me = ((hk >> 32) << 32) | (unsigned long long)(i + 1);
     uint32_t h = (uint32_t)hk & (T - 1);
     for (;;) {
@@ -1361,12 +1443,12 @@ __device__ __forceinline__ uint32_t merge_twins_impl(const WaveMem& m, Rec<W>* c
       }
       h = (h + 1) & (T - 1);
     }
-    __hip_atomic_fetch_min(&tab[h].mi, crec[i].minidx & ~kSkip, __ATOMIC_RELAXED,
+    __hip_atomic_fetch_min(&tab[h].mi, me_.minidx & ~kSkip, __ATOMIC_RELAXED,
                            __HIP_MEMORY_SCOPE_WORKGROUP);
-    const uint32_t rp = crec[i].rep;
+    const uint32_t rp = me_.rep;
     if (rp != kNone)
       __hip_atomic_fetch_min(&tab[h].rep, rp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-    add_wg(&tab[h].ksum, crec[i].ksum);
+    add_wg(&tab[h].ksum, me_.ksum);
     __hip_atomic_fetch_min(&tab[h].first, i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     // every probe that compares against this entry's bitset has its answer
     // from the CAS above; the bitset itself is left untouched
@@ -1375,26 +1457,43 @@ __device__ __forceinline__ uint32_t merge_twins_impl(const WaveMem& m, Rec<W>* c
   wave_mem_wait();
   uint32_t n = 0, nbr = 0;
   uint64_t best = ~0ull;
+  // entry and slot of the next chunk are loaded before this chunk is written
+  // (at or below the entries read so far)
+  struct Next {
+    uint32_t first, mi, rep;
+    uint64_t ksum, a[W];
+  } nt;
+  auto load = [&](uint32_t i) {
+    nt.first = kNone;
+    nt.mi = kNone;
+    nt.rep = kNone;
+    nt.ksum = 0;
+#pragma unroll
+    for (int w = 0; w < W; ++w) nt.a[w] = 0;
+    if (i < len) {
+      const uint32_t h = ld_wg(&crec[i].minidx);
+#pragma unroll
+      for (int w = 0; w < W; ++w) nt.a[w] = crec[i].a[w];
+      nt.first = ld_wg(&tab[h].first);
+      nt.mi = ld_wg(&tab[h].mi);
+      nt.rep = ld_wg(&tab[h].rep);
+      nt.ksum = ld_wg(&tab[h].ksum);
+    }
+  };
+  load(lane);
   for (uint32_t base = 0; base < len; base += kWave) {
     const uint32_t i = base + lane;
-    bool keep = false;
-    uint32_t h = 0;
-    uint64_t a[W];
-#pragma unroll
-    for (int w = 0; w < W; ++w) a[w] = 0;
-    if (i < len) {
-      h = ld_wg(&crec[i].minidx);
-      keep = ld_wg(&tab[h].first) == i;
-#pragma unroll
-      for (int w = 0; w < W; ++w) a[w] = crec[i].a[w];
-    }
+    const Next me_ = nt;
+    const bool keep = i < len && me_.first == i;
+    load(i + kWave);
+    const uint64_t* a = me_.a;
     const uint64_t km = ballot(keep);
     const uint32_t pos = n + lanes_below(km);
     uint32_t rp = kNone;
     wave_mem_wait();  // every lane has read its entry before any is overwritten
     if (keep) {
-      rp = ld_wg(&tab[h].rep);
-      const uint32_t mi = ld_wg(&tab[h].mi);
+      rp = me_.rep;
+      const uint32_t mi = me_.mi;
       // ordered lists: a group whose smallest member is not its pushable one
       // is non-maximal whenever pushed (that member contains it and comes
       // first), here and below; it becomes excluded, so that every pushable
@@ -1402,7 +1501,7 @@ __device__ __forceinline__ uint32_t merge_twins_impl(const WaveMem& m, Rec<W>* c
       if (ordered && rp != kNone && rp != mi) rp = kNone;
       crec[pos].minidx = mi;
       crec[pos].rep = rp;
-      crec[pos].ksum = ld_wg(&tab[h].ksum);
+      crec[pos].ksum = me_.ksum;
 #pragma unroll
       for (int w = 0; w < W; ++w) crec[pos].a[w] = a[w];
       if (rp != kNone) {
@@ -1413,25 +1512,28 @@ __device__ __forceinline__ uint32_t merge_twins_impl(const WaveMem& m, Rec<W>* c
     nbr += __popcll(ballot(rp != kNone));
     n += __popcll(km);
   }
-  wave_mem_wait();
-  best_child = (wave_min_pair(best));
-  cbranch = nbr;
-  return n;
+  lds_flat_fence();
+  return ListOut{wave_min_pair(best), n, nbr, 0, 0};
 }
 
 // The list and the table are reached through generic pointers (flat_
 // accesses) while an LDS list is read and written with ds_ accesses
-// elsewhere: fenced on both sides.
+// elsewhere: merge_leaf fences on both sides.
 template <int W>
 __device__ __forceinline__ uint32_t merge_twins(const WaveMem& m, Rec<W>* crec, uint32_t len,
                                                 uint32_t& lds_top, uint64_t& hbm_top,
                                                 uint64_t& best_child, uint32_t& cbranch,
                                                 bool ordered) {
-  lds_flat_fence();
-  const uint32_t n = merge_twins_impl<W>(m, crec, len, lds_top, hbm_top, best_child, cbranch,
-                                         ordered);
-  lds_flat_fence();
-  return n;
+  uint32_t T = 64;
+  while (T < 2 * len) T <<= 1;
+  uint32_t tier = 1;
+  uint64_t tb = 0;
+  const uint64_t tab = arena_take(m, lds_top, hbm_top, (uint64_t)T * sizeof(MergeSlot), tier, tb);
+  if (tab == 0) return len;
+  const ListOut o = merge_leaf<W>(crec, len, (MergeSlot*)tab, T, ordered);
+  best_child = uni64(o.best);
+  cbranch = uni(o.cbranch);
+  return uni(o.len);
 }
 
 // Reduce a node's list before its first push.  With minrep the smallest
@@ -1457,11 +1559,15 @@ __device__ __forceinline__ uint32_t merge_twins(const WaveMem& m, Rec<W>* crec, 
 // is read from its lane, and the dominators are chosen and applied round by
 // round (a dropped entry is never chosen, and a chosen one is never dropped
 // later: a later dominator has no more bits and, if equal, a later lane).
-template <int W, bool LDS = false>
-__device__ __forceinline__ uint32_t reduce_chunk(const Params& P, Rec<W>* recs, uint32_t len, int K,
-                                                 uint32_t minrep, uint64_t& best,
-                                                 uint32_t& cbranch, Counters& ctr) {
+template <int W, bool LDS>
+MBE_LEAF ListOut reduce_chunk(Rec<W>* recs_, uint32_t len_, uint32_t K_, uint32_t minrep_,
+                              uint32_t dom_skip_) {
   const uint32_t lane = lane_id();
+  const uint32_t len = uni(len_), minrep = uni(minrep_);
+  const int K = (int)uni(K_);
+  const bool dom_skip = uni(dom_skip_) != 0;
+  Rec<W>* recs = uni_ptr(recs_);
+  uint64_t best;
   const bool valid = lane < len;
   uint32_t mi = kNone, rp = kNone;
   uint64_t ks = 0, a[W];
@@ -1494,7 +1600,7 @@ __device__ __forceinline__ uint32_t reduce_chunk(const Params& P, Rec<W>* recs, 
   }
   // dominators, round by round: the excluded lane of largest key that is
   // neither dropped nor chosen yet
-  bool drop = false, chosen = false, sk = P.dom_skip && push && mi < rp;
+  bool drop = false, chosen = false, sk = dom_skip && push && mi < rp;
   for (int r = 0; r < K; ++r) {
     const uint32_t mx = wave_max_u32(excl && !drop && !chosen ? key : 0u);
     if (mx == 0) break;
@@ -1514,21 +1620,20 @@ __device__ __forceinline__ uint32_t reduce_chunk(const Params& P, Rec<W>* recs, 
   }
   const uint64_t vm = ballot(valid), pm = ballot(push), dm = ballot(drop);
   uint64_t sm = ballot(sk);
-  if (!P.dom_skip) sm = 0;
+  if (!dom_skip) sm = 0;
   const uint64_t km = vm & ~dm;
   sm &= km;
   const uint64_t bm = pm & km & ~sm;  // pushes left at this node
   if (dm == 0 && sm == 0) {
     // nothing dropped or marked: the list stands as it is
-    if (P.dom_skip) {
+    if (dom_skip) {
       best = bm ? (((uint64_t)read_lane(rp, (uint32_t)__builtin_ctzll(bm)) << 32) |
                    (uint32_t)__builtin_ctzll(bm))
                 : ~0ull;
     } else {
       best = wave_min_pair(lane_bit(bm) ? (((uint64_t)rp << 32) | lane) : ~0ull);
     }
-    cbranch = __popcll(bm);
-    return len;
+    return ListOut{best, len, (uint32_t)__popcll(bm), 0, 0};
   }
   const bool keep = lane_bit(km);
   sk = lane_bit(sm);
@@ -1551,7 +1656,7 @@ __device__ __forceinline__ uint32_t reduce_chunk(const Params& P, Rec<W>* recs, 
     }
   }
   wave_mem_wait();
-  if (P.dom_skip) {  // ordered list: the first push is the first such position
+  if (dom_skip) {  // ordered list: the first push is the first such position
     if (bm) {
       const uint32_t l = (uint32_t)__builtin_ctzll(bm);
       best = ((uint64_t)read_lane(rp, l) << 32) | (uint32_t)__popcll(km & ((1ull << l) - 1ull));
@@ -1561,31 +1666,19 @@ __device__ __forceinline__ uint32_t reduce_chunk(const Params& P, Rec<W>* recs, 
   } else {
     best = wave_min_pair(lane_bit(bm) ? (((uint64_t)rp << 32) | pos) : ~0ull);
   }
-  cbranch = __popcll(bm);
-  if (P.profile) {
-    ctr.dropped += __popcll(dm);
-    ctr.skipped += __popcll(sm);
-  }
-  return __popcll(km);
+  return ListOut{best, (uint32_t)__popcll(km), (uint32_t)__popcll(bm), (uint32_t)__popcll(dm),
+                 (uint32_t)__popcll(sm)};
 }
 
+// The same for a list of more than 64 entries.
 template <int W>
-__device__ __forceinline__ uint32_t reduce_list(const Params& P, const WaveMem& m, Rec<W>* recs, uint32_t len,
-                                uint64_t& best, uint32_t& cbranch, Counters& ctr) {
+MBE_LEAF ListOut reduce_long(Rec<W>* recs_, uint32_t len_, uint32_t K_, uint32_t minrep_,
+                             uint32_t dom_skip_) {
   const uint32_t lane = lane_id();
-  const int K = P.dom_k < kMaxDom ? P.dom_k : kMaxDom;
-  if (K <= 0 || best == ~0ull || len < 2 || len < (uint32_t)P.reduce_min || len >= (1u << 20))
-    return len;
-  const uint64_t tr = P.profile ? cycles() : 0;
-  if (len <= (uint32_t)kWave) {
-    const uint32_t n =
-        in_lds(m, recs)
-            ? reduce_chunk<W, true>(P, recs, len, K, (uint32_t)(best >> 32), best, cbranch, ctr)
-            : reduce_chunk<W, false>(P, recs, len, K, (uint32_t)(best >> 32), best, cbranch, ctr);
-    if (P.profile) ctr.c_reduce += cycles() - tr;
-    return n;
-  }
-  const uint32_t minrep = (uint32_t)(best >> 32);
+  const uint32_t len = uni(len_), minrep = uni(minrep_);
+  const int K = (int)uni(K_);
+  const bool dom_skip = uni(dom_skip_) != 0;
+  Rec<W>* recs = uni_ptr(recs_);
   lds_flat_fence();  // a list in LDS is reached below through generic pointers
   // dominators: every lane keeps its two largest keys = (popcount + 1) << 20 |
   // ~pos among the excluded entries of one pass over the list, and K maxima
@@ -1619,10 +1712,6 @@ __device__ __forceinline__ uint32_t reduce_list(const Params& P, const WaveMem& 
 #pragma unroll
   for (int w = 0; w < W; ++w) dom[w] = lane < (uint32_t)nd ? recs[dposv].a[w] : 0;
   lds_flat_fence();
-  if (nd == 0 && !P.dom_skip) {
-    if (P.profile) ctr.c_reduce += cycles() - tr;
-    return len;
-  }
   uint32_t out = 0, nbr = 0, ndrop = 0, nskip = 0;
   uint64_t nb = ~0ull;
   // compaction writes only below the chunk it reads, so the next chunk is
@@ -1663,7 +1752,7 @@ __device__ __forceinline__ uint32_t reduce_list(const Params& P, const WaveMem& 
         sk = sk || push;
       }
     }
-    if (!P.dom_skip) sk = false;
+    if (!dom_skip) sk = false;
     const bool keep = valid && !drop;
     const uint64_t km = ballot(keep);
     const uint32_t pos = out + lanes_below(km);
@@ -1685,14 +1774,28 @@ __device__ __forceinline__ uint32_t reduce_list(const Params& P, const WaveMem& 
     out += __popcll(km);
   }
   lds_flat_fence();
-  best = (wave_min_pair(nb));
-  cbranch = nbr;
+  return ListOut{wave_min_pair(nb), out, nbr, ndrop, nskip};
+}
+
+template <int W>
+__device__ __forceinline__ uint32_t reduce_list(const Params& P, const WaveMem& m, Rec<W>* recs, uint32_t len,
+                                uint64_t& best, uint32_t& cbranch, Counters& ctr) {
+  const int K = P.dom_k < kMaxDom ? P.dom_k : kMaxDom;
+  if (K <= 0 || best == ~0ull || len < 2 || len < (uint32_t)P.reduce_min || len >= (1u << 20))
+    return len;
+  const uint64_t tr = P.profile ? cycles() : 0;
+  const uint32_t minrep = (uint32_t)(best >> 32), sk = P.dom_skip != 0;
+  const ListOut o = len > (uint32_t)kWave ? reduce_long<W>(recs, len, (uint32_t)K, minrep, sk)
+                    : in_lds(m, recs)     ? reduce_chunk<W, true>(recs, len, (uint32_t)K, minrep, sk)
+                                          : reduce_chunk<W, false>(recs, len, (uint32_t)K, minrep, sk);
+  best = uni64(o.best);
+  cbranch = uni(o.cbranch);
   if (P.profile) {
-    ctr.dropped += ndrop;
-    ctr.skipped += nskip;
+    ctr.dropped += uni(o.dropped);
+    ctr.skipped += uni(o.skipped);
     ctr.c_reduce += cycles() - tr;
   }
-  return out;
+  return uni(o.len);
 }
 
 // Whether sharing a node is worthwhile now: the top-level vertices are all
@@ -1905,7 +2008,8 @@ __device__ __forceinline__ void dfs(const Params& P, const WaveMem& m, uint32_t 
   const bool prune = P.prune != 0;
   const int64_t* voff = m.g->v_off;
   const uint32_t swapped = m.g->swapped;
-  uint32_t depth = 0, tick = 0;
+  uint32_t depth = 0;
+  uint32_t work = 0;  // since the last look at sharing, in chunks of 64 entries pushed over
   // this subtree's result counters, in scalar registers until it ends
   uint64_t l_nodes = 0, l_nonmax = 0, l_max = 0, l_hsum = 0, l_hxor = 0;
   auto flush = [&]() {
@@ -1916,7 +2020,6 @@ __device__ __forceinline__ void dfs(const Params& P, const WaveMem& m, uint32_t 
     ctr.hxor ^= l_hxor;
   };
   for (;;) {
-    ++tick;
     // one wall-clock read per push: a push over a long list costs far more
     if (P.budget != 0 && past_deadline(P, m.deadline)) {
       ctr.abandoned++;
@@ -1932,9 +2035,13 @@ __device__ __forceinline__ void dfs(const Params& P, const WaveMem& m, uint32_t 
       F = frame_get(m, fb + depth);
       continue;
     }
-    if (P.late_share && !P.list && (tick & 31u) == 0 &&
-        late_share<W, KL_R, C_R>(P, m, gw, nL, nC, ta, F, fb, depth, ctr))
-      continue;  // the current frame was handed over: F.cur is now kNone
+    work += 1 + F.len / kWave;
+    if (P.late_share && !P.list && work >= 32u) {
+      // by work done, not by pushes: 32 pushes over a hub's list take milliseconds
+      work = 0;
+      if (late_share<W, KL_R, C_R>(P, m, gw, nL, nC, ta, F, fb, depth, ctr))
+        continue;  // the current frame was handed over: F.cur is now kNone
+    }
     R_t* recs = (R_t*)F.rec;
     const uint32_t xpos = F.cur, xidx = F.curidx;
     if (P.count_bytes) {
@@ -2226,6 +2333,43 @@ __device__ __forceinline__ void run_items(const Params& P, const WaveMem& m, uin
   }
 }
 
+// The root list of a task: one record per candidate with its bitset over L;
+// clears the candidate index map.
+template <int Wt>
+MBE_LEAF void build_list(Rec<Wt>* brec_, const uint32_t* L_, uint32_t nL_, const uint32_t* C_,
+                         uint32_t nC_, uint32_t next_id_, const uint64_t* kV_, int32_t* cmap_,
+                         const int64_t* off_, const uint32_t* adj_, uint32_t* s_off_,
+                         int64_t* s_start_) {
+  const uint32_t lane = lane_id();
+  auto* brec = uni_ptr(brec_);
+  const uint32_t *L = uni_ptr(L_), *C = uni_ptr(C_), *adj = uni_ptr(adj_);
+  const uint64_t* kV = uni_ptr(kV_);
+  const int64_t* off = uni_ptr(off_);
+  int32_t* cmap = uni_ptr(cmap_);
+  const uint32_t nL = uni(nL_), nC = uni(nC_), next_id = uni(next_id_);
+#pragma unroll 4
+  for (uint32_t i = lane; i < nC; i += kWave) {
+    brec[i].minidx = i;
+    brec[i].rep = i >= next_id ? i : kNone;
+    brec[i].ksum = kV[C[i]];
+#pragma unroll
+    for (int w = 0; w < Wt; ++w) brec[i].a[w] = 0ull;
+  }
+  wave_mem_wait();
+  for_each_edge(L, nL, off, adj, uni_ptr(s_off_), uni_ptr(s_start_),
+                [&](const uint32_t* j, const uint32_t* w, const bool* ok) {
+    int32_t p[kEdges];
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) p[e] = ok[e] ? ld_wg(cmap + w[e]) : 0;
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e)
+      if (p[e] < 0) or_wg(&brec[-p[e] - 1].a[j[e] >> 6], 1ull << (j[e] & 63));
+  });
+  wave_mem_wait();
+  for (uint32_t i = lane; i < nC; i += kWave) st_wg(cmap + C[i], 0);
+  wave_mem_wait();
+}
+
 // Build the root list of a task (entry i starts as candidate i alone:
 // minidx = i, rep = i if i >= next_id else kNone, bitset of L ∩ N(C[i]) with
 // Wt words, zero-padded beyond |L|; with one-word bitsets the candidates are
@@ -2253,21 +2397,7 @@ __device__ __forceinline__ void enumerate_task(const Params& P, const WaveMem& m
   hbm_top = (uint64_t)nC * sizeof(R_t);
   if (P.count_bytes) ctr.blist += (uint64_t)nC * sizeof(R_t);
   R_t* brec = (R_t*)braw;
-  for (uint32_t i = lane; i < nC; i += kWave) {
-    brec[i].minidx = i;
-    brec[i].rep = i >= next_id ? i : kNone;
-    brec[i].ksum = m.kC[i];
-#pragma unroll
-    for (int w = 0; w < Wt; ++w) brec[i].a[w] = 0ull;
-  }
-  wave_mem_wait();
-  for_each_edge(L, nL, g.u_off, g.u_adj, m.s_off, m.s_start, [&](uint32_t j, uint32_t w) {
-    int32_t p = ld_wg(cmap + w);
-    if (p < 0) or_wg(&brec[-p - 1].a[j >> 6], 1ull << (j & 63));
-  });
-  wave_mem_wait();
-  for (uint32_t i = lane; i < nC; i += kWave) st_wg(cmap + m.C[i], 0);
-  wave_mem_wait();
+  build_list<Wt>(brec, L, nL, m.C, nC, next_id, g.kV, cmap, g.u_off, g.u_adj, m.s_off, m.s_start);
   // group twins (not in list mode: its R' lists need one entry per candidate)
   uint32_t len = nC;
   const uint64_t list_addr = braw;
@@ -2397,6 +2527,115 @@ __device__ __forceinline__ Prefix prefix_common(const DevGraph& g, const WaveMem
   return p;
 }
 
+// Counts |N(w) ∩ L| of the task L in cmap, then the 2-hop set (U, ascending)
+// split into the closure R and the candidates C (next_id of them below vk).
+struct RootOut {
+  uint64_t edges;
+  uint32_t nU2, nR, nC, next_id;
+};
+MBE_LEAF uint64_t count_edges(const uint32_t* L_, uint32_t nL_, const int64_t* off_,
+                              const uint32_t* adj_, int32_t* cmap_, uint64_t* bm0_, uint64_t* bm1_,
+                              uint32_t* s_off_, int64_t* s_start_) {
+  const uint32_t* L = uni_ptr(L_);
+  const uint32_t nL = uni(nL_);
+  const int64_t* off = uni_ptr(off_);
+  const uint32_t* adj = uni_ptr(adj_);
+  int32_t* cmap = uni_ptr(cmap_);
+  uint64_t *bm0 = uni_ptr(bm0_), *bm1 = uni_ptr(bm1_);
+  const uint64_t root_edges = for_each_edge(L, nL, off, adj, uni_ptr(s_off_), uni_ptr(s_start_),
+                                            [&](const uint32_t*, const uint32_t* w, const bool* ok) {
+    int32_t old[kEdges];
+    uint64_t o0[kEdges];
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) {
+      old[e] = 1;
+      if (ok[e]) old[e] = add_wg(cmap + w[e], 1);
+    }
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) {
+      o0[e] = 1;
+      if (old[e] == 0) o0[e] = or_wg(bm0 + (w[e] >> 6), 1ull << (w[e] & 63));
+    }
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e)
+      if (o0[e] == 0) or_wg(bm1 + (w[e] >> 12), 1ull << ((w[e] >> 6) & 63));
+  });
+  wave_mem_wait();
+  return root_edges;
+}
+MBE_LEAF RootOut split_two_hop(const int32_t* cmap_, uint64_t* bm0_, uint64_t* bm1_, uint32_t nW1_,
+                               uint32_t* U_, uint32_t* R_, uint32_t* C_, uint32_t nL_,
+                               uint32_t vk_) {
+  const uint32_t lane = lane_id();
+  const int32_t* cmap = uni_ptr(cmap_);
+  uint64_t *bm0 = uni_ptr(bm0_), *bm1 = uni_ptr(bm1_);
+  const uint32_t nW1 = uni(nW1_), nL = uni(nL_), vk = uni(vk_);
+  uint32_t *U = uni_ptr(U_), *R = uni_ptr(R_), *C = uni_ptr(C_);
+  // sorted extraction of the 2-hop set; clears the bitmaps
+  uint32_t nU2 = 0;
+  for (uint32_t b1 = 0; b1 < nW1; b1 += kWave) {
+    uint32_t i1 = b1 + lane;
+    uint64_t s = i1 < nW1 ? ld_wg(bm1 + i1) : 0ull;
+    if (s) st_wg(bm1 + i1, 0ull);
+    uint64_t nz = ballot(s != 0);
+    while (nz) {
+      uint32_t src = first_lane(nz);
+      nz &= nz - 1;
+      uint64_t sw = read_lane64(s, src);
+      uint32_t w0 = (b1 + src) * 64 + lane;
+      uint64_t word = ((sw >> lane) & 1ull) ? ld_wg(bm0 + w0) : 0ull;
+      if (word) st_wg(bm0 + w0, 0ull);
+      uint32_t pc = __popcll(word);
+      uint32_t incl = wave_incl_scan32(pc);
+      uint32_t pos = nU2 + incl - pc;
+      while (word) {
+        uint32_t b = __builtin_ctzll(word);
+        word &= word - 1;
+        U[pos++] = w0 * 64 + b;
+      }
+      nU2 += read_lane(incl, kWave - 1);
+    }
+  }
+  wave_mem_wait();
+  // R = closure, C = the rest (src/IterFinderGpu.cu:794,830-834); the counts of
+  // kEdges chunks are gathered at a time
+  uint32_t nR = 0, nC = 0, next_id = 0;
+  for (uint32_t base = 0; base < nU2; base += kEdges * kWave) {
+    uint32_t w[kEdges], c[kEdges];
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) {
+      const uint32_t i = base + e * kWave + lane;
+      w[e] = i < nU2 ? U[i] : 0;
+    }
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) {
+      const uint32_t i = base + e * kWave + lane;
+      c[e] = i < nU2 ? (uint32_t)ld_wg(cmap + w[e]) : 0;
+    }
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) {
+      const bool valid = base + e * kWave + lane < nU2;
+      const bool isR = valid && c[e] == nL, isC = valid && c[e] != nL;
+      const uint64_t mR = ballot(isR), mC = ballot(isC);
+      if (isR) R[nR + lanes_below(mR)] = w[e];
+      if (isC) C[nC + lanes_below(mC)] = w[e];
+      next_id += __popcll(ballot(isC && w[e] < vk));
+      nR += __popcll(mR);
+      nC += __popcll(mC);
+    }
+  }
+  wave_mem_wait();
+  return RootOut{0, nU2, nR, nC, next_id};
+}
+
+// Whether the waves will run out of top-level vertices soon and the queue is
+// short.
+__device__ __forceinline__ bool hungry(const Params& P) {
+  const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / kWave);
+  return uni64(ld_dev(P.s.root_next)) + waves >= roots_total(P.s) &&
+         (long long)uni64(ld_dev(P.s.queued)) < (long long)P.share_queue;
+}
+
 // One task S = t.v[0..k).  For k > 1, `pre` is the common neighbourhood of
 // S[0..k-1) (prefix_common).
 template <int WMAX>
@@ -2433,68 +2672,16 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
   phase(ctr, P.profile, 1, t0);
   // 2-hop counts
   int32_t* cmap = m.cmap;
-  uint64_t* bm0 = m.bm0;
-  uint64_t* bm1 = m.bm1;
-  // B(root) = 4 (deg(S) + sum of deg(u), u in L)
-  const uint64_t root_edges = for_each_edge(L, nL, g.u_off, g.u_adj, m.s_off, m.s_start,
-                                            [&](uint32_t, uint32_t w) {
-    int32_t old = add_wg(cmap + w, 1);
-    if (old == 0) {
-      uint64_t o0 = or_wg(bm0 + (w >> 6), 1ull << (w & 63));
-      if (o0 == 0) or_wg(bm1 + (w >> 12), 1ull << ((w >> 6) & 63));
-    }
-  });
+  const uint64_t root_edges = uni64(count_edges(L, nL, g.u_off, g.u_adj, cmap, m.bm0, m.bm1, m.s_off,
+                                                m.s_start));
   if (P.count_bytes) {
     ctr.balg += 4ull * (sdeg + root_edges);
     ctr.blist += 4ull * (sdeg + root_edges);
   }
   ctr.edges += root_edges;
-  wave_mem_wait();
   phase(ctr, P.profile, 2, t0);
-  // sorted extraction of the 2-hop set with its counts; clears the bitmaps
-  uint32_t nU2 = 0;
-  for (uint32_t b1 = 0; b1 < P.w.nW1; b1 += kWave) {
-    uint32_t i1 = b1 + lane;
-    uint64_t s = i1 < P.w.nW1 ? ld_wg(bm1 + i1) : 0ull;
-    if (s) st_wg(bm1 + i1, 0ull);
-    uint64_t nz = ballot(s != 0);
-    while (nz) {
-      uint32_t src = first_lane(nz);
-      nz &= nz - 1;
-      uint64_t sw = read_lane64(s, src);
-      uint32_t w0 = (b1 + src) * 64 + lane;
-      uint64_t word = ((sw >> lane) & 1ull) ? ld_wg(bm0 + w0) : 0ull;
-      if (word) st_wg(bm0 + w0, 0ull);
-      uint32_t pc = __popcll(word);
-      uint32_t incl = wave_incl_scan32(pc);
-      uint32_t pos = nU2 + incl - pc;
-      while (word) {
-        uint32_t b = __builtin_ctzll(word);
-        word &= word - 1;
-        uint32_t id = w0 * 64 + b;
-        m.U[pos] = id;
-        m.Ucnt[pos] = (uint32_t)ld_wg(cmap + id);
-        ++pos;
-      }
-      nU2 += read_lane(incl, kWave - 1);
-    }
-  }
-  wave_mem_wait();
-  // R = closure, C = the rest (src/IterFinderGpu.cu:794,830-834)
-  uint32_t nR = 0, nC = 0, next_id = 0;
-  for (uint32_t base = 0; base < nU2; base += kWave) {
-    uint32_t i = base + lane;
-    bool valid = i < nU2;
-    uint32_t w = valid ? m.U[i] : 0, c = valid ? m.Ucnt[i] : 0;
-    bool isR = valid && c == nL, isC = valid && c != nL;
-    uint64_t mR = ballot(isR), mC = ballot(isC);
-    if (isR) m.R[nR + lanes_below(mR)] = w;
-    if (isC) m.C[nC + lanes_below(mC)] = w;
-    next_id += __popcll(ballot(isC && w < vk));
-    nR += __popcll(mR);
-    nC += __popcll(mC);
-  }
-  wave_mem_wait();
+  const RootOut ro = split_two_hop(cmap, m.bm0, m.bm1, P.w.nW1, m.U, m.R, m.C, nL, vk);
+  const uint32_t nU2 = uni(ro.nU2), nR = uni(ro.nR), nC = uni(ro.nC), next_id = uni(ro.next_id);
   // canonicity
   bool canonical;
   if (k == 1) {
@@ -2521,6 +2708,7 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
     }
   }
   auto clear_cmap = [&]() {
+#pragma unroll 4
     for (uint32_t i = lane; i < nU2; i += kWave) st_wg(cmap + m.U[i], 0);
     wave_mem_wait();
   };
@@ -2568,12 +2756,19 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
   // context slots is free and large enough
   uint32_t share_ctx = kNone;
   // (whether its reduced root list fits the slot is decided once it is built)
-  if (rule && P.share && !P.list && W <= (uint32_t)WMAX) share_ctx = free_ctx(P, gw);
+  // and other waves are, or will soon be, short of work: while there are more
+  // top-level vertices unclaimed than waves a task runs where it is, and late
+  // sharing hands out the rest of it when they run out.  (The light vertices of
+  // a 1.5M-edge graph spent 56% of their time publishing lists nobody waited
+  // for.)
+  const bool hg = rule && hungry(P);
+  if (hg && P.share && !P.list && W <= (uint32_t)WMAX) share_ctx = free_ctx(P, gw);
   const bool share = share_ctx != kNone;
   // a large task with no context slot free: its children are recomputed by
   // other waves (recompute, the reference's LargeToTiny) or, by default, the
   // task runs here and late sharing hands its frames out when waves run dry
-  const bool recompute = rule && k < P.max_prefix && (P.recompute || !P.share || P.list);
+  const bool recompute =
+      rule && k < P.max_prefix && ((P.recompute && hg) || !P.share || P.list);
   if (!share && (recompute || (must && k < kMaxPrefix))) {
     // children S + [C[i]], i >= next_id, each recomputed by its wave
     const unsigned long long ne = (rest + kChunk - 1) / kChunk;
@@ -2628,7 +2823,6 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
   for (uint32_t i = lane; i < nR; i += kWave) st_wg(cmap + m.R[i], 0);
   for (uint32_t i = lane; i < nC; i += kWave) {
     st_wg(cmap + m.C[i], -(int32_t)(i + 1));
-    m.kC[i] = g.kV[m.C[i]];
   }
   for (uint32_t j = lane; j < nL; j += kWave) {
     m.kL[j] = g.kU[L[j]];

@@ -172,6 +172,24 @@ __device__ __forceinline__ const __attribute__((address_space(3))) T* as_lds(con
   return (const __attribute__((address_space(3))) T*)p;
 }
 
+// A generic pointer known to address device memory: global_ accesses.
+template <class T>
+__device__ __forceinline__ __attribute__((address_space(1))) T* as_glb(T* p) {
+  return (__attribute__((address_space(1))) T*)p;
+}
+// A pointer that is the same in every lane, in scalar registers.
+template <class T>
+__device__ __forceinline__ T* uni_ptr(T* p) {
+  return (T*)uni64((uint64_t)p);
+}
+
+// The work of a node or a task is split into leaf functions that are not
+// inlined: each is compiled once with registers of its own.  As one body the
+// kernel spilled 1,700 scalar and 1,500 vector registers and did not fit the
+// instruction cache by a factor of ten.  Uniform arguments arrive in vector
+// registers and are moved to scalar ones first.
+#define MBE_LEAF __device__ __attribute__((noinline))
+
 // Ordering of this wave's own memory operations across its lanes.  Within a
 // work-group (one CU) the hardware keeps them coherent, so this is a
 // compiler-level fence (no cache maintenance is emitted).
