@@ -36,10 +36,13 @@ mbe::Scratch scratch_layout(uint32_t nV, uint32_t dmaxV, uint64_t arena_bytes,
 
 // Control counters live kCtlStride u64 (256 bytes) apart so that polling one
 // never contends with atomics on another; the shards' head/tail pairs follow.
-enum CtlSlot { C_ROOT_NEXT = 0, C_WORK_LEFT, C_QUEUED, C_LIST_CURSOR, C_DEFERRED, C_WIDE_N,
+enum CtlSlot { C_ROOT_NEXT = 0, C_WORK_LEFT, C_LIST_CURSOR, C_DEFERRED, C_WIDE_N,
                C_DEADLINE,  // absolute deadline of the run (wall clock), shared by both passes
-               C_QCTL = 8, C_NSLOTS = 8 + 2 * mbe::kShards };
+               C_QCTL = 8, C_IDLE = C_QCTL + 2 * mbe::kShards,
+               C_NSLOTS = C_IDLE + mbe::kIdleWords * mbe::kIdleStride / mbe::kCtlStride };
 constexpr uint64_t kCtlWords = (uint64_t)C_NSLOTS * mbe::kCtlStride;
+// The waves' mail words follow (each wave clears its own before it waits).
+constexpr uint64_t kMailWords = (uint64_t)mbe::kIdleWords * 64 * mbe::kIdleStride;
 
 typedef void (*KernelFn)(mbe::Params);
 struct KernelChoice {

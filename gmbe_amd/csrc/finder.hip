@@ -359,7 +359,7 @@ struct gmbe_finder {
   unsigned long long* qseq = nullptr;
   uint64_t qcap = 0;
   // control counters, each on its own 256-byte line (kCtlStride u64 apart):
-  // root_next, work_left, queued, list_cursor, n_deferred, then per-shard head/tail
+  // root_next, work_left, list_cursor, n_deferred, .., per-shard head/tail, idle bitmap
   unsigned long long* ctl = nullptr;
   unsigned long long* acc = nullptr;  // in ctl's allocation, with the graph table
   unsigned long long* out = nullptr;  // pinned: the words of run_result
@@ -506,7 +506,7 @@ static int gmbe_finder_create_impl(const gmbe_graph* g, int sel, int bound_heigh
   }
   rc = f->dg.upload(*g);
   // control block, result block and graph table in one allocation
-  const size_t b_ctl = kCtlWords * 8, b_acc = ((size_t)mbe::A_COUNT * 8 + 255) & ~(size_t)255;
+  const size_t b_ctl = (kCtlWords + kMailWords) * 8, b_acc = ((size_t)mbe::A_COUNT * 8 + 255) & ~(size_t)255;
   if (rc == GMBE_OK && hipMalloc(&f->ctl, b_ctl + b_acc + sizeof(mbe::DevGraph)) != hipSuccess)
     rc = set_error(GMBE_ERR_NOMEM, "control block");
   if (rc == GMBE_OK && hipHostMalloc((void**)&f->out, (kOutCtl + mbe::A_COUNT) * 8,
@@ -615,7 +615,8 @@ static int gmbe_finder_execute_impl(gmbe_finder* f, gmbe_result* res) {
   P.s.root_next = f->ctl + C_ROOT_NEXT * kCtlStride;
   P.s.work_left = f->ctl + C_WORK_LEFT * kCtlStride;
   P.s.qctl = f->ctl + C_QCTL * kCtlStride;
-  P.s.queued = f->ctl + C_QUEUED * kCtlStride;
+  P.s.idle = f->ctl + C_IDLE * kCtlStride;
+  P.s.mail = f->ctl + kCtlWords;
   P.list_cursor = f->ctl + C_LIST_CURSOR * kCtlStride;
   P.s.n_deferred = f->ctl + C_DEFERRED * kCtlStride;
   P.s.deadline_word = f->ctl + C_DEADLINE * kCtlStride;

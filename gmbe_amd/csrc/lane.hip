@@ -167,7 +167,7 @@ int Lane::alloc(Engine* e, const LaneCaps& c, const LaneKnobs& k) {
   LANE_TRY(hipMalloc(&root_base, (ng + kLaneClasses) * 8));
   LANE_TRY(hipMalloc(&order, ng * 4));
   LANE_TRY(hipMalloc(&per_graph, ng * kPerGraph * 8));
-  LANE_TRY(hipMalloc(&ctl, kCtlWords * 8));
+  LANE_TRY(hipMalloc(&ctl, (kCtlWords + kMailWords) * 8));
   LANE_TRY(hipMalloc(&acc, mbe::A_COUNT * 8));
   LANE_TRY(hipMalloc(&deferred, knobs.deferred_cap * sizeof(mbe::Task)));
   // the arrays of a full lane plus the 16-byte alignment of each of the nine
@@ -398,7 +398,8 @@ mbe::Params Lane::params(bool wide) const {
   P.s.root_next = ctl + C_ROOT_NEXT * kCtlStride;
   P.s.work_left = ctl + C_WORK_LEFT * kCtlStride;
   P.s.qctl = ctl + C_QCTL * kCtlStride;
-  P.s.queued = ctl + C_QUEUED * kCtlStride;
+  P.s.idle = ctl + C_IDLE * kCtlStride;
+  P.s.mail = ctl + kCtlWords;
   P.list_cursor = ctl + C_LIST_CURSOR * kCtlStride;
   P.s.n_deferred = ctl + C_DEFERRED * kCtlStride;
   P.s.deadline_word = ctl + C_DEADLINE * kCtlStride;  // one absolute deadline for both passes

@@ -43,6 +43,8 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr int kMaxPrefix = 8;              // task capacity (vertices)
 constexpr int kShards = 32;                // independent queue rings
 constexpr int kCtlStride = 32;             // u64 between control counters (256 B)
+constexpr int kIdleWords = 64;             // waves that can wait for a wake-up: 64 per word
+constexpr int kIdleStride = 8;             // u64 between those words (64 B)
 constexpr int kMaxW = 16;                  // widest bitset (|L| <= 1024)
 constexpr int kMainW = 4;                  // widest bitset of the main kernel
 constexpr int kMaxDom = 16;                // dominators tried per list (reduce_list)
@@ -98,7 +100,8 @@ struct Sched {
   uint32_t* q;                    // kShards rings of kEntryWords-word entries
   unsigned long long* qseq;       // per-slot sequence numbers
   unsigned long long* qctl;       // per shard: head, tail (kCtlStride u64 apart)
-  unsigned long long* queued;     // entries pushed and not yet popped (a hint)
+  unsigned long long* idle;       // a bit per waiting wave: kIdleWords words, kIdleStride apart
+  unsigned long long* mail;       // a word per wave that can wait, kIdleStride apart
   unsigned long long qcap;        // slots per shard, power of two
   unsigned long long n_roots;     // top-level vertices of this run (sample)
   const unsigned long long* n_roots_dev;  // if set, the count is read here instead
@@ -404,63 +407,103 @@ __device__ __forceinline__ uint64_t for_each_edge(const uint32_t* L, uint32_t nL
 constexpr int kChunk = 24;      // children per entry
 constexpr int kEntryWords = 32; // hdr, prefix[7], children[24]
 
-// Longest nap of a wave without work, in units of 2,048 cycles.  A run ends, and
-// a shared subtree starts, one nap late at worst; shorter naps poll more often.
-constexpr uint32_t kMaxNap = 8;
-
-__device__ __forceinline__ void backoff(uint32_t& n) {
-  for (uint32_t i = 0; i < n; ++i) __builtin_amdgcn_s_sleep(32);
-  n = n < kMaxNap ? n * 2 : kMaxNap;
-}
-
 __device__ __forceinline__ unsigned long long* shard_head(const Sched& s, uint32_t sh) {
   return s.qctl + (uint64_t)(2 * sh) * kCtlStride;
 }
 __device__ __forceinline__ unsigned long long* shard_tail(const Sched& s, uint32_t sh) {
-  return s.qctl + (uint64_t)(2 * sh + 1) * kCtlStride;
+  return shard_head(s, sh) + 1;  // the same line: one look reads both
 }
 __device__ __forceinline__ uint64_t slot_of(const Sched& s, uint32_t sh, unsigned long long pos) {
   return (uint64_t)sh * s.qcap + (pos & (s.qcap - 1));
 }
 
-// Pop one entry into `word` (lane l < 32 holds word l), scanning the shards
-// from `home`.
-__device__ __forceinline__ bool queue_pop(const Sched& s, uint32_t& word, uint32_t home) {
+// Waiting without polling.  What the waves of a starved run did to each other
+// was the largest cost of sharing: a few thousand of them reading the queue's
+// counters over and over delay the atomics of those who publish and pop (60-80
+// ns each on one address, and the planted-block graph takes 10^6 entries).  So a
+// wave without work sets its bit in a bitmap, looks at everything once more, and
+// then reads nothing but a word of its own; who publishes entries wakes as many
+// waves as there are entries, by clearing their bits and writing their words.
+// Either the waiting wave's last look sees the entries or the publisher's look
+// at the bitmap, which follows the push, sees the wave.
+
+constexpr uint32_t kMailEnd = 64;  // nothing is left; 1 + sh: look at shard sh
+
+__device__ __forceinline__ unsigned long long* mail_of(const Sched& s, uint64_t wave) {
+  return s.mail + wave * kIdleStride;
+}
+// Wake up to n waiting waves with the message `msg`.
+__device__ __forceinline__ void wake(const Params& P, uint32_t n, uint32_t msg) {
   const uint32_t lane = lane_id();
-  if ((long long)uni64(ld_dev(s.queued)) <= 0) return false;
-  unsigned long long got = ~0ull;
-  uint32_t gsh = 0;
+  unsigned long long* word = P.s.idle + (uint64_t)lane * kIdleStride;
+  const uint64_t v = ld_dev(word);
+  if (ballot(v != 0) == 0) return;
+  const uint32_t pc = __popcll(v), before = wave_incl_scan32(pc) - pc;
+  uint64_t take = 0;
+  if (before < n) {
+    uint64_t rest = v;
+    for (uint32_t i = before; i < n && rest != 0; ++i) rest &= rest - 1;
+    take = v ^ rest;
+  }
+  if (take != 0) {
+    take &= __hip_atomic_fetch_and(word, (unsigned long long)~take, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+    while (take != 0) {
+      st_dev(mail_of(P.s, (uint64_t)lane * 64 + __builtin_ctzll(take)), msg);
+      take &= take - 1;
+    }
+  }
+}
+// Whether the wave's home shard holds fewer entries than its part of
+// share_queue: the other shards are taken to look alike.
+__device__ __forceinline__ bool home_short(const Sched& s, uint32_t home, int share_queue) {
+  const long long lim = share_queue > kShards ? share_queue / kShards : 1;
+  const unsigned long long v = ld_dev(shard_head(s, home) + (lane_id() & 1u));
+  return (long long)(read_lane64(v, 1) - read_lane64(v, 0)) < lim;
+}
+
+// Pop one entry of shard sh into `word` (lane l < 32 holds word l).
+__device__ __forceinline__ bool queue_pop_shard(const Sched& s, uint32_t& word, uint32_t sh) {
+  const uint32_t lane = lane_id();
+  const unsigned long long v = ld_dev(shard_head(s, sh) + (lane & 1u));
+  unsigned long long h = read_lane64(v, 0), got = ~0ull;
+  if (h >= read_lane64(v, 1)) return false;
   if (lane == 0) {
-    for (uint32_t i = 0; i < (uint32_t)kShards && got == ~0ull; ++i) {
-      const uint32_t sh = (home + i) & (kShards - 1);
-      unsigned long long h = ld_dev(shard_head(s, sh));
-      for (int tries = 0; tries < 4; ++tries) {
-        unsigned long long tl = ld_dev(shard_tail(s, sh));
-        if (h >= tl) break;
-        if (__hip_atomic_compare_exchange_strong(shard_head(s, sh), &h, h + 1, __ATOMIC_RELAXED,
-                                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
-          got = h;
-          gsh = sh;
-          break;
-        }
+    for (int tries = 0; tries < 4; ++tries) {
+      if (__hip_atomic_compare_exchange_strong(shard_head(s, sh), &h, h + 1, __ATOMIC_RELAXED,
+                                               __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+        got = h;
+        break;
       }
+      if (h >= ld_dev(shard_tail(s, sh))) break;
     }
-    if (got != ~0ull) {
-      __hip_atomic_fetch_add(s.queued, (unsigned long long)-1ll, __ATOMIC_RELAXED,
-                             __HIP_MEMORY_SCOPE_AGENT);
-      const uint64_t slot = slot_of(s, gsh, got);
-      while (ld_dev(s.qseq + slot) != got + 1) __builtin_amdgcn_s_sleep(1);
-    }
+    if (got != ~0ull)
+      while (ld_dev(s.qseq + slot_of(s, sh, got)) != got + 1) __builtin_amdgcn_s_sleep(1);
   }
   got = uni64(got);
   if (got == ~0ull) return false;
-  gsh = uni(gsh);
   wave_drain();
-  const uint64_t slot = slot_of(s, gsh, got);
+  const uint64_t slot = slot_of(s, sh, got);
   word = lane < (uint32_t)kEntryWords ? ld_dev(s.q + slot * kEntryWords + lane) : 0u;
   wave_drain();
   if (lane == 0) st_dev(s.qseq + slot, got + s.qcap);
   return true;
+}
+// The same from any shard: one look at all of them, then those that hold
+// entries from `home` on.
+__device__ __forceinline__ bool queue_pop_any(const Sched& s, uint32_t& word, uint32_t home) {
+  const uint32_t lane = lane_id();
+  const unsigned long long v = ld_dev(shard_head(s, lane & (kShards - 1)) + lane / kShards);
+  const uint64_t t = ((uint64_t)shfl_xor32((uint32_t)(v >> 32), kShards) << 32) |
+                     shfl_xor32((uint32_t)v, kShards);
+  uint32_t mask = (uint32_t)ballot(lane < (uint32_t)kShards && v < t);
+  while (mask != 0) {
+    const uint32_t turned = home ? (mask >> home) | (mask << (kShards - home)) : mask;
+    const uint32_t sh = (home + (uint32_t)__builtin_ctz(turned)) & (kShards - 1);
+    if (queue_pop_shard(s, word, sh)) return true;
+    mask &= ~(1u << sh);
+  }
+  return false;
 }
 
 // Reserve ne consecutive positions in one shard, trying `home` first.
@@ -494,9 +537,10 @@ __device__ __forceinline__ bool queue_reserve(const Sched& s, uint32_t home, uin
 
 // Push the children prefix+[cand[i]], i < n, as ceil(n / kChunk) entries.
 // All or nothing: false (nothing pushed) when the queue lacks room.
-__device__ __forceinline__ bool queue_push_children(const Sched& s, const Task& prefix, int k,
+__device__ __forceinline__ bool queue_push_children(const Params& P, const Task& prefix, int k,
                                     const uint32_t* cand, uint32_t n, uint32_t& n_entries,
                                     uint32_t home) {
+  const Sched& s = P.s;
   uint32_t lane = lane_id();
   const uint32_t ne = (n + kChunk - 1) / kChunk;
   n_entries = ne;
@@ -524,9 +568,7 @@ __device__ __forceinline__ bool queue_push_children(const Sched& s, const Task& 
     if (e < ne && w == 0) st_dev(s.qseq + slot_of(s, sh, start + e), start + e + 1);
   }
   wave_drain();
-  if (lane == 0)
-    __hip_atomic_fetch_add(s.queued, (unsigned long long)ne, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+  wake(P, ne, 1 + sh);
   return true;
 }
 
@@ -541,21 +583,66 @@ __device__ __forceinline__ unsigned long long roots_total(const Sched& s) {
 // every unit has finished (the gc/lc/tc protocol of
 // src/IterFinderGpu.cu:978-986,1020-1034 collapsed into one outstanding-work
 // counter), 1 for an entry (in `word`), 2 for a root task (in `t`, `k`).
-__device__ __forceinline__ int next_work(const Params& P, uint32_t& word, Task& t, int& k, uint32_t home,
-                         uint64_t deadline) {
+// pay() settles the wave's credits before it first waits and returns whether the
+// run has ended with them.
+template <class Pay>
+__device__ __forceinline__ int next_work(const Params& P, uint32_t& word, Task& t, int& k, uint64_t gw,
+                         uint64_t deadline, Pay&& pay) {
   const Sched& s = P.s;
-  uint32_t lane = lane_id();
-  uint32_t nap = 1;
+  const uint32_t lane = lane_id(), home = (uint32_t)(gw & (kShards - 1));
+  uint32_t look = home;  // the shard looked at first
+  bool paid = false;
   const unsigned long long n_roots = roots_total(s);
   for (;;) {
     if (past_deadline(P, deadline)) return 0;  // leave what is queued: the run is cut short
-    if (queue_pop(s, word, home)) return 1;
+    if (queue_pop_shard(s, word, look)) return 1;
     unsigned long long r = ~0ull;
     if (lane == 0 && ld_dev(s.root_next) < n_roots) {
       r = __hip_atomic_fetch_add(s.root_next, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     r = uni64(r);
-    if (r != ~0ull && r < n_roots) {
+    if (r == ~0ull || r >= n_roots) {
+      if (queue_pop_any(s, word, home)) return 1;
+      if (!paid && pay()) return 0;
+      paid = true;
+      // a wave past the bitmap waits without it
+      const bool can = gw < (uint64_t)kIdleWords * 64;
+      unsigned long long* mail = mail_of(s, can ? gw : 0);
+      unsigned long long* idle = s.idle + (can ? gw / 64 : 0) * kIdleStride;
+      const unsigned long long bit = can ? 1ull << (gw & 63) : 0ull;
+      if (lane == 0 && can) {
+        st_dev(mail, 0ull);
+        mem_drain();
+        __hip_atomic_fetch_or(idle, bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+      wave_drain();
+      uint32_t msg = 0;
+      for (uint32_t naps = 0; msg == 0; ++naps) {
+        if ((naps & 63u) == 0) {
+          // the look that follows the bit (and now and then another one)
+          const bool end = uni64(ld_dev(s.work_left)) == 0;
+          if (end || queue_pop_any(s, word, home)) {
+            unsigned long long old = bit;
+            if (lane == 0 && can)
+              old = __hip_atomic_fetch_and(idle, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (end) return 0;
+            // woken meanwhile: another wave has to have that
+            if (can && !(uni64(old) & bit)) wake(P, 1, 1 + home);
+            return 1;
+          }
+        }
+        if (past_deadline(P, deadline)) return 0;
+        __builtin_amdgcn_s_sleep(16);
+        if (can) msg = (uint32_t)uni64(ld_dev(mail));
+      }
+      if (msg == kMailEnd) return 0;
+      // a word written late for an earlier wait leaves the bit set: take it back
+      if (lane == 0 && ((ld_dev(idle) & bit) != 0))
+        __hip_atomic_fetch_and(idle, ~bit, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      look = msg - 1;
+      continue;
+    }
+    {
       if (s.root_tasks) {
         uint32_t w = lane < (uint32_t)kMaxPrefix ? s.root_tasks[r].v[lane] : kNone;
         k = 0;
@@ -585,16 +672,54 @@ __device__ __forceinline__ int next_work(const Params& P, uint32_t& word, Task& 
       k = 1;
       return 2;
     }
-    unsigned long long left = uni64(lane == 0 ? ld_dev(s.work_left) : 0ull);
-    if (left == 0) return 0;
-    backoff(nap);
   }
 }
 
-__device__ __forceinline__ void work_done(const Params& P) {
-  if (lane_id() == 0)
-    __hip_atomic_fetch_add(P.s.work_left, (unsigned long long)-1ll, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+// The wave finished a unit: credited here, paid by work_pay (or spent on units
+// that it publishes).
+__device__ __forceinline__ void work_done(SmallCallPtr sc) {
+  if (lane_id() == 0) {
+    sc->credit += 1;
+    sc->gcredit += 1;
+  }
+  wave_mem_wait();
+}
+// Outstanding units of the run, and of graph gid, grow by n: the wave's credits
+// first.  (The counters are never below what is outstanding.)
+__device__ __forceinline__ void work_add(const Sched& s, unsigned long long* per_graph, uint32_t gid,
+                                         SmallCallPtr sc, uint32_t n) {
+  if (lane_id() == 0) {
+    const uint32_t c = sc->credit, u = c < n ? c : n;
+    sc->credit = c - u;
+    if (n > u)
+      __hip_atomic_fetch_add(s.work_left, (unsigned long long)(n - u), __ATOMIC_RELAXED,
+                             __HIP_MEMORY_SCOPE_AGENT);
+    if (per_graph) {
+      const uint32_t cg = sc->gcredit, ug = cg < n ? cg : n;
+      sc->gcredit = cg - ug;
+      if (n > ug)
+        __hip_atomic_fetch_add(per_graph + (uint64_t)gid * kPerGraph + G_LEFT,
+                               (unsigned long long)(n - ug), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+  wave_mem_wait();
+}
+// Pays what is credited; true when that was the last outstanding work (the
+// waiting waves are told).
+__device__ __forceinline__ bool work_pay(const Params& P, SmallCallPtr sc) {
+  const uint32_t n = uni(sc->credit);
+  if (n == 0) return false;
+  unsigned long long left = 0;
+  if (lane_id() == 0) {
+    left = __hip_atomic_fetch_add(P.s.work_left, (unsigned long long)(-(long long)n),
+                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    sc->credit = 0;
+  }
+  wave_mem_wait();
+  if (uni64(left) != n) return false;
+  wake(P, kIdleWords * 64, kMailEnd);
+  return true;
 }
 
 // ---------------------------------------------------------------------------
@@ -744,11 +869,13 @@ __device__ __forceinline__ void small_setup(const Params& P, const WaveMem& m, u
   if (lane_id() == 0) {
     auto* sc = as_lds(m.sc);
     sc->root_next = P.s.root_next;
-    sc->queued = P.s.queued;
+    sc->head = shard_head(P.s, (uint32_t)(gw & (kShards - 1)));
     sc->n_roots = n_roots;
+    sc->credit = 0;
+    sc->gcredit = 0;
     sc->deadline = P.budget != 0 ? m.deadline : 0;
     sc->save = (uint32_t*)(P.w.base + gw * P.w.slab + P.w.o_save);
-    sc->share_queue = P.share_queue;
+    sc->share_queue = P.share_queue > kShards ? P.share_queue / kShards : 1;
     sc->share_len = P.late_share > 0 ? (uint32_t)P.late_share : 0u;
     sc->dom_k = (uint32_t)(P.dom_k < kMaxDom ? (P.dom_k > 0 ? P.dom_k : 0) : kMaxDom);
     sc->prune = P.prune != 0;
@@ -798,15 +925,6 @@ __device__ __forceinline__ uint64_t arena_take(const WaveMem& m, uint32_t& lds_t
     return (uint64_t)(m.arena + hbm_top);
   }
   return 0;
-}
-
-__device__ __forceinline__ uint64_t wave_min64(uint64_t x) {
-  for (int s = 32; s > 0; s >>= 1) {
-    uint32_t lo = shfl_xor32((uint32_t)x, s), hi = shfl_xor32((uint32_t)(x >> 32), s);
-    uint64_t y = ((uint64_t)hi << 32) | lo;
-    x = y < x ? y : x;
-  }
-  return x;
 }
 
 // Task-level arrays a stack machine reads: hash keys of L (by L index) and
@@ -1111,7 +1229,8 @@ template <int W, bool KL_R, bool C_R>
 MBE_LEAF bool publish_leaf(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t gid_,
                            const Rec<W>* root_, uint32_t len_, uint32_t nL_, uint32_t nC_,
                            uint32_t nbits_, uint64_t sumR0_, const uint64_t* kL_,
-                           const uint32_t* C_, uint32_t min_rep_, uint32_t min_items_) {
+                           const uint32_t* C_, uint32_t min_rep_, uint32_t min_items_,
+                           SmallCallPtr sc) {
   const Params& P = leaf_params(kp);
   const uint32_t gw = uni(gw_), ctx = uni(ctx_), gid = uni(gid_), len = uni(len_), nL = uni(nL_),
                  nC = uni(nC_), nbits = uni(nbits_), min_rep = uni(min_rep_),
@@ -1171,10 +1290,7 @@ MBE_LEAF bool publish_leaf(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t gi
     if (lane == 0) st_dev(&h->refs, 0ull);
     return false;
   }
-  if (lane == 0)
-    __hip_atomic_fetch_add(s.work_left, (unsigned long long)ne, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-  graph_work(P, gid, (long long)ne);
+  work_add(s, P.per_graph, gid, sc, ne);
   // fill the entries: item j goes to entry j / 15, slot j % 15
   uint32_t j0 = 0;
   for (uint32_t base = 0; base < len; base += kWave) {
@@ -1211,21 +1327,19 @@ MBE_LEAF bool publish_leaf(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t gi
   wave_drain();
   for (uint32_t e = lane; e < ne; e += kWave) st_dev(s.qseq + slot_of(s, sh, start + e), start + e + 1);
   wave_drain();
-  if (lane == 0)
-    __hip_atomic_fetch_add(s.queued, (unsigned long long)ne, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+  wake(P, ne, 1 + sh);
   return true;
 }
 
 template <int W, bool KL_R, bool C_R>
-__device__ __forceinline__ bool publish_list(const Params& P, uint64_t gw, uint32_t ctx,
+__device__ __forceinline__ bool publish_list(const Params& P, const WaveMem& m, uint64_t gw, uint32_t ctx,
                                              uint32_t gid, const Rec<W>* root, uint32_t len,
                                              uint32_t nL, uint32_t nC, uint32_t nbits,
                                              uint64_t sumR0, const TaskArrays& src,
                                              uint32_t min_rep = 0, uint32_t min_items = 1) {
   return uni((uint32_t)publish_leaf<W, KL_R, C_R>(kernel_params(), (uint32_t)gw, ctx, gid, root,
                                                   len, nL, nC, nbits, sumR0, src.kL, src.C,
-                                                  min_rep, min_items)) != 0;
+                                                  min_rep, min_items, as_lds(m.sc))) != 0;
 }
 
 // Publish a node of small_dfs (at most 64 entries, one per lane) as this wave's
@@ -1234,7 +1348,7 @@ __device__ __forceinline__ bool publish_list(const Params& P, uint64_t gw, uint3
 // order, all that a push looks at.
 MBE_LEAF bool publish_small(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t gid_, uint32_t nL_,
                             uint64_t a0, uint64_t ks, uint64_t key,
-                            const __attribute__((address_space(3))) SmallCall* sc) {
+                            SmallCallPtr sc) {
   const Params& P = leaf_params(kp);
   const uint32_t gw = uni(gw_), ctx = uni(ctx_), gid = uni(gid_), nL = uni(nL_);
   const uint64_t L = uni64(sc->sh_L), alive = uni64(sc->sh_alive), push = uni64(sc->sh_push),
@@ -1273,10 +1387,7 @@ MBE_LEAF bool publish_small(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t g
     if (lane == 0) st_dev(&h->refs, 0ull);
     return false;
   }
-  if (lane == 0)
-    __hip_atomic_fetch_add(s.work_left, (unsigned long long)ne, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
-  graph_work(P, gid, (long long)ne);
+  work_add(s, P.per_graph, gid, sc, ne);
   // item j (the j-th bit of todo) goes to entry j / 15, slot j % 15
   if (lane_bit(todo)) {
     const uint32_t j = lanes_below(todo);
@@ -1297,9 +1408,7 @@ MBE_LEAF bool publish_small(uint64_t kp, uint32_t gw_, uint32_t ctx_, uint32_t g
   wave_drain();
   if (lane < ne) st_dev(s.qseq + slot_of(s, sh, start + lane), start + lane + 1);
   wave_drain();
-  if (lane == 0)
-    __hip_atomic_fetch_add(s.queued, (unsigned long long)ne, __ATOMIC_RELAXED,
-                           __HIP_MEMORY_SCOPE_AGENT);
+  wake(P, ne, 1 + sh);
   return true;
 }
 
@@ -1807,8 +1916,7 @@ __device__ __forceinline__ uint32_t share_wanted(const Params& P, uint64_t gw, u
                          (P.count_bytes ? (uint64_t)nC * 4 : 0);
   if (bytes > P.w.ctx_bytes) return kNone;
   if (uni64(ld_dev(P.s.root_next)) < roots_total(P.s)) return kNone;
-  const long long depth = (long long)uni64(ld_dev(P.s.queued));
-  if (depth >= (long long)P.share_queue) return kNone;
+  if (!home_short(P.s, (uint32_t)(gw & (kShards - 1)), P.share_queue)) return kNone;
   return free_ctx(P, gw);
 }
 
@@ -1888,7 +1996,7 @@ __device__ __forceinline__ bool child_node(const Params& P, const WaveMem& m, ui
                                 : kNone;
         if (cx != kNone) {
           uint64_t tq = P.profile ? cycles() : 0;
-          shared = publish_list<1, false, C_R>(P, gw, cx, graph_id(P, m), dst, dlen, nb, nC, nb, sumR, tc);
+          shared = publish_list<1, false, C_R>(P, m, gw, cx, graph_id(P, m), dst, dlen, nb, nC, nb, sumR, tc);
           if (P.profile) ctr.c_publish += cycles() - tq;
         }
         if (shared) {
@@ -1936,7 +2044,7 @@ __device__ __forceinline__ bool child_node(const Params& P, const WaveMem& m, ui
                           : kNone;
   if (cx != kNone) {
     uint64_t tq = P.profile ? cycles() : 0;
-    bool ok = publish_list<W, KL_R, C_R>(P, gw, cx, graph_id(P, m), crec, clen, nL, nC, nb, sumR, ta);
+    bool ok = publish_list<W, KL_R, C_R>(P, m, gw, cx, graph_id(P, m), crec, clen, nL, nC, nb, sumR, ta);
     if (P.profile) ctr.c_publish += cycles() - tq;
     if (ok) {
       ctr.splits++;
@@ -1961,7 +2069,7 @@ __device__ __forceinline__ bool late_share(const Params& P, const WaveMem& m, ui
   // cheap gate first: the top-level vertices are all claimed and the queue is
   // short; then pick the shallowest frame with pushes left
   if (uni64(ld_dev(P.s.root_next)) < roots_total(P.s)) return false;
-  if ((long long)uni64(ld_dev(P.s.queued)) >= (long long)P.share_queue) return false;
+  if (!home_short(P.s, (uint32_t)(gw & (kShards - 1)), P.share_queue)) return false;
   uint32_t at = kNone;
   Frame S;
   const uint32_t scan = depth < 4u ? depth : 4u;
@@ -1981,7 +2089,7 @@ __device__ __forceinline__ bool late_share(const Params& P, const WaveMem& m, ui
   const uint32_t cx = share_wanted(P, gw, nL, nC, S.len, W);
   if (cx == kNone) return false;
   uint64_t tq = P.profile ? cycles() : 0;
-  const bool ok = publish_list<W, KL_R, C_R>(P, gw, cx, graph_id(P, m), (const Rec<W>*)S.rec, S.len, nL, nC,
+  const bool ok = publish_list<W, KL_R, C_R>(P, m, gw, cx, graph_id(P, m), (const Rec<W>*)S.rec, S.len, nL, nC,
                                              S.nbits, S.sumR, ta, S.curidx, 2);
   if (P.profile) ctr.c_publish += cycles() - tq;
   if (!ok) return false;
@@ -2429,7 +2537,7 @@ __device__ __forceinline__ void enumerate_task(const Params& P, const WaveMem& m
   const uint64_t need = sizeof(CtxHdr) + (uint64_t)len * sizeof(R_t) + (uint64_t)nL * 8 +
                         (P.count_bytes ? (uint64_t)nC * 4 : 0);
   if (share_ctx != kNone && need <= P.w.ctx_bytes &&
-      publish_list<Wt, false, false>(P, gw, share_ctx, graph_id(P, m), (const R_t*)list_addr, len, nL, nC, nL,
+      publish_list<Wt, false, false>(P, m, gw, share_ctx, graph_id(P, m), (const R_t*)list_addr, len, nL, nC, nL,
                                      sumR, lta)) {
     ctr.splits++;
     phase(ctr, P.profile, 6, t0);
@@ -2530,7 +2638,6 @@ __device__ __forceinline__ Prefix prefix_common(const DevGraph& g, const WaveMem
 // Counts |N(w) ∩ L| of the task L in cmap, then the 2-hop set (U, ascending)
 // split into the closure R and the candidates C (next_id of them below vk).
 struct RootOut {
-  uint64_t edges;
   uint32_t nU2, nR, nC, next_id;
 };
 MBE_LEAF uint64_t count_edges(const uint32_t* L_, uint32_t nL_, const int64_t* off_,
@@ -2625,15 +2732,15 @@ MBE_LEAF RootOut split_two_hop(const int32_t* cmap_, uint64_t* bm0_, uint64_t* b
     }
   }
   wave_mem_wait();
-  return RootOut{0, nU2, nR, nC, next_id};
+  return RootOut{nU2, nR, nC, next_id};
 }
 
 // Whether the waves will run out of top-level vertices soon and the queue is
 // short.
-__device__ __forceinline__ bool hungry(const Params& P) {
+__device__ __forceinline__ bool hungry(const Params& P, uint64_t gw) {
   const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / kWave);
   return uni64(ld_dev(P.s.root_next)) + waves >= roots_total(P.s) &&
-         (long long)uni64(ld_dev(P.s.queued)) < (long long)P.share_queue;
+         home_short(P.s, (uint32_t)(gw & (kShards - 1)), P.share_queue);
 }
 
 // One task S = t.v[0..k).  For k > 1, `pre` is the common neighbourhood of
@@ -2761,7 +2868,7 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
   // sharing hands out the rest of it when they run out.  (The light vertices of
   // a 1.5M-edge graph spent 56% of their time publishing lists nobody waited
   // for.)
-  const bool hg = rule && hungry(P);
+  const bool hg = rule && hungry(P, gw);
   if (hg && P.share && !P.list && W <= (uint32_t)WMAX) share_ctx = free_ctx(P, gw);
   const bool share = share_ctx != kNone;
   // a large task with no context slot free: its children are recomputed by
@@ -2776,7 +2883,7 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
       __hip_atomic_fetch_add(P.s.work_left, ne, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     graph_work(P, t.gid, (long long)ne);
     uint32_t pushed = 0;
-    if (queue_push_children(P.s, t, k, m.C + next_id, rest, pushed,
+    if (queue_push_children(P, t, k, m.C + next_id, rest, pushed,
                             (uint32_t)(gw & (kShards - 1)))) {
       ctr.splits++;
       count_root(sumL, sumR);

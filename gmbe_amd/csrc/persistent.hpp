@@ -51,26 +51,50 @@ void mbe_persistent(Params P) {
   Task t;
   int k = 0;
   uint32_t word = 0;
+  // The results and finished units of one graph are kept until a unit of
+  // another graph comes or the wave goes idle: its counters are one address for
+  // every wave that works on the graph.
+  const uint32_t no_graph = 0xFFFFFFFFu;
+  uint32_t on = no_graph;
+  auto pay_graph = [&]() {
+    if (!P.per_graph || on == no_graph) return;
+    flush_graph(P, c, on);
+    const uint32_t n = uni(as_lds(m.sc)->gcredit);
+    if (n != 0) graph_work(P, on, -(long long)n);
+    on = no_graph;
+  };
   for (;;) {
     uint64_t tw = P.profile ? cycles() : 0;
-    int kind = next_work(P, word, t, k, (uint32_t)(gw & (kShards - 1)), m.deadline);
+    int kind = next_work(P, word, t, k, gw, m.deadline, [&]() {
+      pay_graph();
+      return work_pay(P, as_lds(m.sc));
+    });
     if (kind == 0) {
+      pay_graph();
+      work_pay(P, as_lds(m.sc));
       // the final wait (nothing left for this wave) goes to the split slot's
       // neighbour so that mid-run waiting and the tail can be told apart
       if (P.profile) c.tail += cycles() - tw;
       break;
     }
     phase(c, P.profile, 0, tw);
-    uint32_t gid;
+    const uint32_t gid = kind == 2 ? t.gid
+                         : (read_lane(word, 0) & kItemKind)
+                             ? uni(ld_dev(&ctx_hdr(P, read_lane(word, 1))->gid))
+                             : child_hdr_gid(read_lane(word, 0));
+    if (P.per_graph && gid != on) {
+      pay_graph();
+      if (lane_id() == 0) as_lds(m.sc)->gcredit = 0;
+      wave_mem_wait();
+      on = gid;
+    }
     if (kind == 2) {
-      gid = t.gid;
       m.g = P.gt + gid;
       Prefix pre{nullptr, 0, 0};
       if (k > 1) pre = prefix_common(*m.g, m, t, k - 1);
       run_task<WMAX>(P, m, t, k, pre, c, gw);
     } else if (read_lane(word, 0) & kItemKind) {
       // items of a shared task context (its header names the graph)
-      gid = uni(ld_dev(&ctx_hdr(P, read_lane(word, 1))->gid));
       m.g = P.gt + gid;
       run_items<WMAX>(P, m, word, c, gw);
     } else {
@@ -79,7 +103,6 @@ void mbe_persistent(Params P) {
       const uint32_t hdr = read_lane(word, 0);
       const int kp = (int)child_hdr_k(hdr);
       const uint32_t cnt = child_hdr_cnt(hdr);
-      gid = child_hdr_gid(hdr);
       m.g = P.gt + gid;
       for (int i = 0; i < kMaxPrefix; ++i) t.v[i] = i < kp ? read_lane(word, 1 + i) : kNone;
       t.gid = gid;
@@ -89,9 +112,7 @@ void mbe_persistent(Params P) {
         run_task<WMAX>(P, m, t, kp + 1, pre, c, gw);
       }
     }
-    if (P.per_graph) flush_graph(P, c, gid);
-    work_done(P);
-    graph_work(P, gid, -1);
+    work_done(as_lds(m.sc));
   }
   if (P.exit_stamps) {
     // the reference's per-SM exit times (src/IterFinderGpu.cu:1038-1041): once

@@ -31,8 +31,9 @@ namespace mbe {
 struct SmallCall {
   // set once per kernel
   const unsigned long long* root_next;  // polled for sharing
-  const unsigned long long* queued;
+  const unsigned long long* head;       // head and tail of the home shard
   unsigned long long n_roots;
+  uint32_t credit, gcredit;  // finished units not yet paid (work_pay), of the run and the graph
   uint64_t deadline;  // wall clock past which the wave stops (0 = none)
   uint32_t* save;     // kSaveWords words of the slab: the stack across a yield
   int32_t share_queue;
@@ -46,6 +47,8 @@ struct SmallCall {
   uint64_t sh_L, sh_alive, sh_push, sh_todo, sh_sumR;
   uint32_t sh_at;
 };
+
+typedef __attribute__((address_space(3))) SmallCall* SmallCallPtr;
 
 enum SmallStatus : uint32_t { SMALL_DONE = 0, SMALL_YIELD = 1, SMALL_CUT = 2 };
 enum SmallResume : uint32_t { SMALL_START = 0, SMALL_RESUME = 1, SMALL_RESUME_SHARED = 2 };
@@ -85,8 +88,8 @@ struct FrameRegs {
 // deadline) is left to the caller (run_small), to which it returns for that.
 template <bool PROF>
 __device__ __attribute__((noinline)) uint32_t small_dfs(
-    __attribute__((address_space(3))) SmallCall* sc, Counters* ctr_, uint32_t nL_, uint32_t resume_,
-    uint64_t a0, uint64_t ks, uint64_t key) {
+    SmallCallPtr sc, Counters* ctr_, uint32_t nL_, uint32_t resume_, uint64_t a0, uint64_t ks,
+    uint64_t key) {
   const uint32_t lane = lane_id();
   const uint32_t nL = uni(nL_), resume = uni(resume_);
   Counters* ctr = (Counters*)uni64((uint64_t)ctr_);
@@ -157,13 +160,14 @@ __device__ __attribute__((noinline)) uint32_t small_dfs(
         break;
       }
       if (share_len != 0) {
-        // one load for both words: are the top-level vertices all claimed, and
-        // is the queue short?
+        // one load for three words: are the top-level vertices all claimed, and
+        // is the home shard's queue short?
         const unsigned long long* q0 = (const unsigned long long*)uni64((uint64_t)sc->root_next);
-        const unsigned long long* q1 = (const unsigned long long*)uni64((uint64_t)sc->queued);
-        const unsigned long long v = ld_dev(lane == 0 ? q0 : q1);
+        const unsigned long long* q1 = (const unsigned long long*)uni64((uint64_t)sc->head);
+        const unsigned long long v = ld_dev(lane == 0 ? q0 : lane == 1 ? q1 : q1 + 1);
         if (read_lane64(v, 0) >= uni64(sc->n_roots) &&
-            (long long)read_lane64(v, 1) < (long long)(int32_t)uni((uint32_t)sc->share_queue)) {
+            (long long)(read_lane64(v, 2) - read_lane64(v, 1)) <
+                (long long)(int32_t)uni((uint32_t)sc->share_queue)) {
           // the shallowest open node with enough left (among the first levels)
           uint32_t at = kShareNone;
           const uint32_t scan = depth < 4u ? depth : 4u;

@@ -114,7 +114,7 @@ static int execute_static_impl(const gmbe_graph* g, int bound_height, int bound_
   const uint64_t b_graph = o;  // what the host copies in
   const uint64_t o_kU = take(nU * 8), o_kV = take(nV * 8);
   const uint64_t o_gt = take(sizeof(mbe::DevGraph));
-  const uint64_t o_ctl = take(kCtlWords * 8), o_acc = take(mbe::A_COUNT * 8);
+  const uint64_t o_ctl = take((kCtlWords + kMailWords) * 8), o_acc = take(mbe::A_COUNT * 8);
   const uint64_t o_q = take(kStaticQcap * mbe::kShards * mbe::kEntryWords * 4);
   const uint64_t o_qseq = take(kStaticQcap * mbe::kShards * 8);
   const uint64_t o_def = take(kStaticDeferred * sizeof(mbe::Task));
@@ -193,7 +193,8 @@ static int execute_static_impl(const gmbe_graph* g, int bound_height, int bound_
   P.s.root_next = ctl + C_ROOT_NEXT * mbe::kCtlStride;
   P.s.work_left = ctl + C_WORK_LEFT * mbe::kCtlStride;
   P.s.qctl = ctl + C_QCTL * mbe::kCtlStride;
-  P.s.queued = ctl + C_QUEUED * mbe::kCtlStride;
+  P.s.idle = ctl + C_IDLE * mbe::kCtlStride;
+  P.s.mail = ctl + kCtlWords;
   P.list_cursor = ctl + C_LIST_CURSOR * mbe::kCtlStride;
   P.s.n_deferred = ctl + C_DEFERRED * mbe::kCtlStride;
   P.s.deferred = (mbe::Task*)(base + o_def);

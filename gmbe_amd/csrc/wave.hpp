@@ -61,17 +61,6 @@ __device__ __forceinline__ uint64_t wave_sum64(uint64_t x) {
   }
   return x;
 }
-__device__ __forceinline__ uint64_t wave_xor64(uint64_t x) {
-  for (int m = 32; m > 0; m >>= 1) {
-    uint32_t lo = shfl_xor32((uint32_t)x, m), hi = shfl_xor32((uint32_t)(x >> 32), m);
-    x ^= ((uint64_t)hi << 32) | lo;
-  }
-  return x;
-}
-__device__ __forceinline__ uint32_t wave_sum32(uint32_t x) {
-  for (int m = 32; m > 0; m >>= 1) x += shfl_xor32(x, m);
-  return x;
-}
 // inclusive prefix sum across the wave
 __device__ __forceinline__ uint32_t wave_incl_scan32(uint32_t x) {
   uint32_t l = lane_id();
@@ -172,11 +161,6 @@ __device__ __forceinline__ const __attribute__((address_space(3))) T* as_lds(con
   return (const __attribute__((address_space(3))) T*)p;
 }
 
-// A generic pointer known to address device memory: global_ accesses.
-template <class T>
-__device__ __forceinline__ __attribute__((address_space(1))) T* as_glb(T* p) {
-  return (__attribute__((address_space(1))) T*)p;
-}
 // A pointer that is the same in every lane, in scalar registers.
 template <class T>
 __device__ __forceinline__ T* uni_ptr(T* p) {
@@ -201,6 +185,13 @@ __device__ __forceinline__ void wave_mem_wait() {
 // that announces it; device-scope release/acquire would instead write back /
 // invalidate the whole L2 of the XCD, which is far too costly per task.
 __device__ __forceinline__ void wave_drain() {
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+  __builtin_amdgcn_s_waitcnt(0);
+  __atomic_signal_fence(__ATOMIC_SEQ_CST);
+}
+
+// The same for code that only some lanes run.
+__device__ __forceinline__ void mem_drain() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
   __builtin_amdgcn_s_waitcnt(0);
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
