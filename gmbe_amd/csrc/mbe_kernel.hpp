@@ -337,14 +337,45 @@ __device__ __forceinline__ uint32_t wave_intersect_count(const uint32_t* A, uint
   return cnt;
 }
 
-// f(j, w, ok) for the edges (L[j], w), w in N(L[j]) over the U->V rows, kEdges
-// per lane at a time (ok marks the ones that exist).  The edges of 64 L
-// vertices are flattened across lanes; each lane finds its vertex by binary
-// search over the 64 prefix offsets kept in LDS (six fixed steps: offsets past
-// the last vertex equal the total, which no edge reaches).  A wave alone on a
-// SIMD hides no latency but its own: with one edge per lane in flight a hub's
-// 30,000-edge pass took 2.5 us per 64 edges.
+// f(at, w, ok) for `total` edges, kEdges per lane at a time (ok marks the ones
+// that exist): run i of adj starts at edge lo_off[i], and lo_start[i] + t is the
+// place of edge t in adj.  Each lane finds its run by binary search over the
+// offsets (fixed steps from `top`, half the runs rounded up to a power of two:
+// offsets past the last run equal the total, which no edge reaches).  A wave
+// alone on a SIMD hides no latency but its own: with one edge per lane in flight
+// a hub's 30,000-edge pass took 2.5 us per 64 edges.
 constexpr int kEdges = 4;
+typedef const __attribute__((address_space(3))) uint32_t* LdsU32;
+typedef const __attribute__((address_space(3))) int64_t* LdsI64;
+template <class F>
+__device__ __forceinline__ void each_run(uint32_t total, uint32_t top, const uint32_t* adj,
+                                         LdsU32 lo_off, LdsI64 lo_start, F&& f) {
+  const uint32_t lane = lane_id();
+  for (uint32_t t0 = 0; t0 < total; t0 += kEdges * kWave) {
+    uint32_t at[kEdges], w[kEdges];
+    bool ok[kEdges];
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) at[e] = 0;
+#pragma unroll
+    for (uint32_t step = top; step > 0; step >>= 1) {
+#pragma unroll
+      for (int e = 0; e < kEdges; ++e) {
+        const uint32_t t = t0 + e * kWave + lane;
+        if (lo_off[at[e] + step] <= t) at[e] += step;
+      }
+    }
+#pragma unroll
+    for (int e = 0; e < kEdges; ++e) {
+      const uint32_t t = t0 + e * kWave + lane;
+      ok[e] = t < total;
+      w[e] = ok[e] ? adj[lo_start[at[e]] + (int64_t)t] : 0;
+    }
+    f(at, w, ok);
+  }
+}
+
+// f(j, w, ok) for the edges (L[j], w), w in N(L[j]) over the U->V rows: the rows
+// of 64 L vertices at a time, flattened across the lanes by each_run.
 template <class F>
 __device__ __forceinline__ uint64_t for_each_edge(const uint32_t* L, uint32_t nL, const int64_t* off,
                                   const uint32_t* adj, uint32_t* s_off, int64_t* s_start, F&& f) {
@@ -367,28 +398,11 @@ __device__ __forceinline__ uint64_t for_each_edge(const uint32_t* L, uint32_t nL
     lo_off[lane] = incl - deg;
     lo_start[lane] = st - (int64_t)(incl - deg);
     wave_mem_wait();
-    for (uint32_t t0 = 0; t0 < total; t0 += kEdges * kWave) {
-      uint32_t at[kEdges], w[kEdges];
-      bool ok[kEdges];
+    each_run(total, 32, adj, lo_off, lo_start, [&](uint32_t* at, const uint32_t* w, const bool* ok) {
 #pragma unroll
-      for (int e = 0; e < kEdges; ++e) at[e] = 0;
-#pragma unroll
-      for (uint32_t step = 32; step > 0; step >>= 1) {
-#pragma unroll
-        for (int e = 0; e < kEdges; ++e) {
-          const uint32_t t = t0 + e * kWave + lane;
-          if (lo_off[at[e] + step] <= t) at[e] += step;
-        }
-      }
-#pragma unroll
-      for (int e = 0; e < kEdges; ++e) {
-        const uint32_t t = t0 + e * kWave + lane;
-        ok[e] = t < total;
-        w[e] = ok[e] ? adj[lo_start[at[e]] + (int64_t)t] : 0;
-        at[e] += base;
-      }
+      for (int e = 0; e < kEdges; ++e) at[e] += base;
       f(at, w, ok);
-    }
+    });
     wave_mem_wait();
   }
   return edges;
@@ -2478,53 +2492,253 @@ MBE_LEAF void build_list(Rec<Wt>* brec_, const uint32_t* L_, uint32_t nL_, const
   wave_mem_wait();
 }
 
-// Build the root list of a task (entry i starts as candidate i alone:
-// minidx = i, rep = i if i >= next_id else kNone, bitset of L ∩ N(C[i]) with
-// Wt words, zero-padded beyond |L|; with one-word bitsets the candidates are
-// then grouped by bitset through a per-wave hash table), then either publish
-// it as a shared context (share) or run the stack machine here.
-template <int Wt>
-__device__ __forceinline__ void enumerate_task(const Params& P, const WaveMem& m, const uint32_t* L, uint32_t nL,
-                               uint32_t nC, uint32_t next_id, uint64_t sumR, uint32_t nR,
-                               Counters& ctr, uint64_t& t0, uint32_t share_ctx, uint64_t gw) {
-  typedef Rec<Wt> R_t;
-  const DevGraph g = *m.g;
+// The root list of a top-level vertex with at most 32 neighbours, in one pass
+// over its two-hop edges and with nothing but the rows and the keys read from
+// memory.  The V side is taken in tiles of LDS that hold one bitset over L per
+// vertex (8, 16 or 32 bits): the part of each row that falls into the tile sets
+// its bits, and a sweep reads the touched vertices back in ascending order.  A
+// vertex with every bit belongs to the closure R; the others are grouped by
+// bitset right away, in a table in LDS, so that one record per group is all that
+// is written.  (A group is what merge_twins would make of its members: their
+// smallest id, their key sum, pushable iff that id is above vk.  Ids take the
+// place of positions among the candidates: only their order matters.)
+//
+// Why: these vertices see thousands of candidates but few different bitsets (6,600
+// edges and 3 to 64 bitsets on the light vertices of the 1.5M-edge power-law graph,
+// 200 and 10 to 30 on a uniform graph), and the general way, whose counts, bitmaps,
+// records and hash table lie in the wave's slab, moves megabytes per vertex there.
+// The light vertices took 227 ms that way and take 8.5 ms this way; the 15,013
+// vertices of a uniform graph of 240,000 edges 2.2 and 1.7 ms.
+//
+// Not done here (kTileNone) when the rows are too thin for their tiles or the
+// groups do not fit the table: the general way takes the vertex then.
+constexpr uint32_t kTileGroups = 224;  // groups the table holds (an index byte each)
+constexpr uint32_t kTileIdx = 512;     // slots of its hash index
+constexpr uint32_t kTileTable = kTileGroups * 16 + kTileIdx;
+constexpr uint32_t kTileLds = kTileTable + 1024;  // smallest list arena it works in
+constexpr uint32_t kTileBuf = 128;                // vertices between sweep and table
+static_assert(kTileBuf * 8 <= kLdsFrames * sizeof(Frame), "the buffer lies over the frames");
+
+enum TileState : uint32_t { kTileNone = 0, kTileList, kTileNonmax };
+struct TileOut {
+  uint32_t state, nR, nC, next_id, len, nbr;
+  uint32_t edges;
+  uint64_t best, sumR;
+};
+
+MBE_LEAF TileOut tile_root(const uint32_t* L_, uint32_t nL_, const int64_t* off_,
+                           const uint32_t* adj_, const uint64_t* kV_, uint32_t nV_, uint32_t vk_,
+                           char* lds_, uint32_t lds_bytes_, Frame* buf_, uint32_t* s_off_,
+                           int64_t* s_start_, Rec<1>* out_) {
   const uint32_t lane = lane_id();
-  int32_t* cmap = m.cmap;
-  uint32_t lds_top = 0;
-  uint64_t hbm_top = 0;
-  // candidate bitsets, one record per candidate, built in the HBM arena
-  if ((uint64_t)nC * sizeof(R_t) > m.arena_bytes) {
-    ctr.overflow++;
-    ctr.ovf_arena++;
-    for (uint32_t i = lane; i < nC; i += kWave) st_wg(cmap + m.C[i], 0);
-    wave_mem_wait();
-    return;
+  const uint32_t nL = uni(nL_), nV = uni(nV_), vk = uni(vk_), lds_bytes = uni(lds_bytes_);
+  const uint32_t *L = uni_ptr(L_), *adj = uni_ptr(adj_);
+  const int64_t* off = uni_ptr(off_);
+  const uint64_t* kV = uni_ptr(kV_);
+  Rec<1>* out = uni_ptr(out_);
+  char* lds = uni_ptr(lds_);
+  auto* eks = as_lds((uint64_t*)lds);
+  auto* emask = as_lds((uint32_t*)(lds + kTileGroups * 8));
+  auto* emi = as_lds((uint32_t*)(lds + kTileGroups * 12));
+  auto* idx = as_lds((uint8_t*)(lds + kTileGroups * 16));
+  auto* idx64 = as_lds((uint64_t*)(lds + kTileGroups * 16));
+  auto* tile = as_lds((uint32_t*)(lds + kTileTable));
+  auto* tile64 = as_lds((uint64_t*)(lds + kTileTable));
+  auto* buf = as_lds((uint64_t*)uni_ptr(buf_));
+  auto* lo_off = as_lds(uni_ptr(s_off_));
+  auto* lo_start = as_lds(uni_ptr(s_start_));
+  TileOut r{kTileNone, 0, 0, 0, 0, 0, 0, ~0ull, 0};
+  // bits per vertex 1 << sh, vertices per tile, rows rounded up to a power of two
+  const uint32_t sh = nL <= 8 ? 3 : nL <= 16 ? 4 : 5;
+  const uint32_t words = (lds_bytes - kTileTable) / 512 * 64, span = (words * 64) >> sh;
+  const uint32_t n_tiles = (nV + span - 1) / span;
+  const uint32_t lg = nL <= 1 ? 0 : 32 - (uint32_t)__builtin_clz(nL - 1);
+  const uint32_t rows = 1u << lg, per = kWave >> lg;  // tiles whose bounds are found at a time
+  const uint32_t j = lane & (rows - 1), b = lane >> lg;
+  int64_t st = 0;
+  uint32_t len = 0;
+  if (j < nL) {
+    const uint32_t u = L[j];
+    st = off[u];
+    len = (uint32_t)(off[u + 1] - st);
   }
-  const uint64_t braw = (uint64_t)m.arena;
-  hbm_top = (uint64_t)nC * sizeof(R_t);
-  if (P.count_bytes) ctr.blist += (uint64_t)nC * sizeof(R_t);
-  R_t* brec = (R_t*)braw;
-  build_list<Wt>(brec, L, nL, m.C, nC, next_id, g.kV, cmap, g.u_off, g.u_adj, m.s_off, m.s_start);
-  // group twins (not in list mode: its R' lists need one entry per candidate)
-  uint32_t len = nC;
-  const uint64_t list_addr = braw;
-  uint64_t best = ~0ull;
-  uint32_t nbr = 0;
-  if (P.group && !P.list && nC > 1) {
-    len = merge_twins<Wt>(m, brec, nC, lds_top, hbm_top, best, nbr, P.dom_skip != 0);
-  }
-  if (len == nC) {
-    // first push: the smallest rep
-    for (uint32_t i = lane; i < len; i += kWave) {
-      const uint32_t rp = brec[i].rep;
-      if (rp != kNone) {
-        const uint64_t c = ((uint64_t)rp << 32) | i;
-        best = c < best ? c : best;
+  r.edges = read_lane(wave_incl_scan32(lane < rows ? len : 0u), kWave - 1);
+  if (n_tiles > 16 + r.edges / 4) return r;
+  lds_flat_fence();  // the list arena may have been reached by flat accesses
+  for (uint32_t i = lane; i < words; i += kWave) tile64[i] = 0;
+  for (uint32_t i = lane; i < kTileIdx / 8; i += kWave) idx64[i] = ~0ull;
+  wave_mem_wait();
+  const uint32_t full = nL == 32 ? ~0u : (1u << nL) - 1u;
+  const uint32_t field = sh == 5 ? ~0u : (1u << (1u << sh)) - 1u;
+  const uint64_t lows = sh == 3 ? 0x0101010101010101ull : sh == 4 ? 0x0001000100010001ull : 0x0000000100000001ull;
+  uint32_t n = 0, seen = 0, taken = 0;
+  uint64_t sumR = 0;
+  bool fits = true, canonical = true;
+  // The next cnt <= 64 vertices of the buffer go to R or to their groups.
+  auto take = [&](uint32_t cnt) {
+    const uint64_t x = buf[(taken + lane) & (kTileBuf - 1)];
+    const uint32_t w = (uint32_t)x, mk = (uint32_t)(x >> 32);
+    const bool valid = lane < cnt, isR = valid && mk == full, isC = valid && mk != full;
+    const uint64_t key = valid ? kV[w] : 0;
+    const uint64_t bR = ballot(isR);
+    r.nR += __popcll(bR);
+    r.nC += cnt - __popcll(bR);
+    r.next_id += __popcll(ballot(isC && w < vk));
+    if (ballot(isR && w < vk) != 0) canonical = false;
+    if (isR) sumR += key;
+    uint32_t h = sh == 3 ? mk : (mk * 0x9E3779B1u) >> 23, e = 255;
+    if (isC) {
+      for (;;) {
+        e = idx[h];
+        if (e == 255 || emask[e] == mk) break;
+        h = (h + 1) & (kTileIdx - 1);
       }
     }
-    best = (wave_min_pair(best));
+    // new bitsets, in the order of their first vertices
+    uint64_t nw = ballot(isC && e == 255);
+    while (nw != 0) {
+      const uint32_t l = (uint32_t)__builtin_ctzll(nw);
+      const uint32_t ml = read_lane(mk, l), wl = read_lane(w, l);
+      uint32_t hl = read_lane(h, l);
+      if (n == kTileGroups) {
+        fits = false;
+        return;
+      }
+      while (uni((uint32_t)idx[hl]) != 255) hl = (hl + 1) & (kTileIdx - 1);
+      if (lane == 0) {
+        idx[hl] = (uint8_t)n;
+        emask[n] = ml;
+        emi[n] = wl;
+        eks[n] = 0;
+      }
+      wave_mem_wait();
+      const bool same = isC && mk == ml;
+      if (same) e = n;
+      nw &= ~ballot(same);
+      ++n;
+    }
+    if (isC)
+      __hip_atomic_fetch_add(eks + e, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    wave_mem_wait();
+    taken += cnt;
+  };
+  uint32_t from = 0;  // where row j goes on
+  for (uint32_t tb = 0; tb < n_tiles; tb += per) {
+    // lane (b, j): the end of tile tb + b in row j
+    const uint64_t end = (uint64_t)(tb + b + 1) * span;
+    uint32_t lo = from, left = len - from;
+    while (ballot(left != 0) != 0) {
+      const uint32_t half = left >> 1;
+      if (left != 0) {
+        if ((uint64_t)adj[st + lo + half] < end) {
+          lo += half + 1;
+          left -= half + 1;
+        } else {
+          left = half;
+        }
+      }
+    }
+    uint32_t start = (uint32_t)__shfl((int)lo, (int)((lane - rows) & (kWave - 1)), kWave);
+    if (b == 0) start = from;
+    from = (uint32_t)__shfl((int)lo, (int)((per - 1) * rows + j), kWave);
+    for (uint32_t bb = 0; bb < per && tb + bb < n_tiles; ++bb) {
+      const int src = (int)((bb * rows + j) & (kWave - 1));
+      const uint32_t s0 = (uint32_t)__shfl((int)start, src, kWave);
+      const uint32_t s1 = (uint32_t)__shfl((int)lo, src, kWave);
+      const uint32_t cnt = lane < nL ? s1 - s0 : 0u;
+      const uint32_t incl = wave_incl_scan32(cnt);
+      const uint32_t total = read_lane(incl, kWave - 1);
+      if (total == 0) continue;
+      lo_off[lane] = incl - cnt;
+      lo_start[lane] = st + (int64_t)s0 - (int64_t)(incl - cnt);
+      wave_mem_wait();
+      const uint32_t v0 = (tb + bb) * span;
+      each_run(total, rows >> 1, adj, lo_off, lo_start,
+               [&](const uint32_t* at, const uint32_t* w, const bool* ok) {
+#pragma unroll
+        for (int e = 0; e < kEdges; ++e) {
+          const uint32_t bit = ((w[e] - v0) << sh) + at[e];
+          if (ok[e])
+            __hip_atomic_fetch_or(tile + (bit >> 5), 1u << (bit & 31), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+      });
+      wave_mem_wait();
+      // the touched vertices, in ascending order, through the buffer
+      for (uint32_t i0 = 0; i0 < words; i0 += kWave) {
+        const uint64_t x = tile64[i0 + lane];
+        if (ballot(x != 0) == 0) continue;
+        if (x != 0) tile64[i0 + lane] = 0;
+        uint64_t y = x | (x >> 1);
+        y |= y >> 2;
+        y |= y >> 4;
+        if (sh > 3) y |= y >> 8;
+        if (sh > 4) y |= y >> 16;
+        y &= lows;
+        const uint32_t pc = __popcll(y), ic = wave_incl_scan32(pc);
+        const uint32_t upto = seen + read_lane(ic, kWave - 1);
+        uint32_t pos = seen + ic - pc;
+        while (seen < upto) {
+          while (y != 0 && pos < taken + kTileBuf) {
+            const uint32_t bit = (uint32_t)__builtin_ctzll(y);
+            y &= y - 1;
+            buf[pos & (kTileBuf - 1)] = ((x >> bit) & field) << 32 | (v0 + (((i0 + lane) * 64 + bit) >> sh));
+            ++pos;
+          }
+          wave_mem_wait();
+          seen = upto < taken + kTileBuf ? upto : taken + kTileBuf;
+          while (fits && seen - taken >= (uint32_t)kWave) take(kWave);
+          if (!fits || !canonical) break;
+        }
+        if (!fits || !canonical) break;
+      }
+      if (!fits) return TileOut{kTileNone, 0, 0, 0, 0, 0, 0, ~0ull, 0};
+      if (!canonical) {
+        r.state = kTileNonmax;
+        return r;
+      }
+    }
   }
+  if (seen != taken) take(seen - taken);
+  if (!fits) return TileOut{kTileNone, 0, 0, 0, 0, 0, 0, ~0ull, 0};
+  r.state = canonical ? kTileList : kTileNonmax;
+  r.len = n;
+  r.sumR = wave_sum_u64(sumR);
+  for (uint32_t base = 0; base < n; base += kWave) {
+    const uint32_t i = base + lane;
+    uint32_t rep = kNone;
+    if (i < n) {
+      const uint32_t mi = emi[i];
+      if (mi > vk) rep = mi;
+      out[i].minidx = mi;
+      out[i].rep = rep;
+      out[i].ksum = eks[i];
+      out[i].a[0] = emask[i];
+    }
+    const uint64_t br = ballot(rep != kNone);
+    if (br != 0 && r.best == ~0ull) {
+      const uint32_t l = (uint32_t)__builtin_ctzll(br);
+      r.best = ((uint64_t)read_lane(rep, l) << 32) | (base + l);
+    }
+    r.nbr += __popcll(br);
+  }
+  wave_mem_wait();
+  return r;
+}
+
+// Reduce a task's root list (`brec`, at the base of the HBM arena; `best` its
+// first push), then either publish it as a shared context (share) or run the
+// stack machine here.
+template <int Wt>
+__device__ __forceinline__ void enumerate_list(const Params& P, const WaveMem& m, Rec<Wt>* brec, uint32_t len,
+                               uint32_t nL, uint32_t nC, uint64_t sumR, uint32_t nR, uint64_t best,
+                               uint32_t nbr, Counters& ctr, uint64_t& t0, uint32_t share_ctx,
+                               uint64_t gw) {
+  typedef Rec<Wt> R_t;
+  const uint32_t lane = lane_id();
+  uint32_t lds_top = 0;
+  uint64_t hbm_top = 0;
+  const uint64_t list_addr = (uint64_t)brec;
   // drop dominated excluded candidates and mark the non-maximal pushes (not in
   // list mode: its R' lists read the root list)
   if (!P.list) len = reduce_list<Wt>(P, m, brec, len, best, nbr, ctr);
@@ -2598,6 +2812,60 @@ __device__ __forceinline__ void enumerate_task(const Params& P, const WaveMem& m
     dfs<Wt, false, false>(P, m, nL, nC, F, lds_top, hbm_top, ctr, ta, root, len, nR, gw, 0);
   }
   phase(ctr, P.profile, 5, t0);
+}
+
+// Build the root list of a task (entry i starts as candidate i alone:
+// minidx = i, rep = i if i >= next_id else kNone, bitset of L ∩ N(C[i]) with
+// Wt words, zero-padded beyond |L|; the candidates are then grouped by bitset
+// through a per-wave hash table) unless tile_root has built it, and enumerate
+// its subtree.
+template <int Wt>
+__device__ __forceinline__ void enumerate_task(const Params& P, const WaveMem& m, const uint32_t* L, uint32_t nL,
+                               uint32_t nC, uint32_t next_id, uint64_t sumR, uint32_t nR,
+                               const TileOut& to, Counters& ctr, uint64_t& t0, uint32_t share_ctx,
+                               uint64_t gw) {
+  typedef Rec<Wt> R_t;
+  const DevGraph g = *m.g;
+  const uint32_t lane = lane_id();
+  int32_t* cmap = m.cmap;
+  const bool tiled = Wt == 1 && to.state != kTileNone;
+  // candidate bitsets, one record per candidate, built in the HBM arena
+  if ((uint64_t)nC * sizeof(R_t) > m.arena_bytes) {
+    ctr.overflow++;
+    ctr.ovf_arena++;
+    if (!tiled)
+      for (uint32_t i = lane; i < nC; i += kWave) st_wg(cmap + m.C[i], 0);
+    wave_mem_wait();
+    return;
+  }
+  R_t* brec = (R_t*)m.arena;
+  uint32_t len = to.len, nbr = to.nbr;
+  uint64_t best = to.best;
+  if (!tiled) {
+    uint32_t lds_top = 0;
+    uint64_t hbm_top = (uint64_t)nC * sizeof(R_t);
+    len = nC;
+    nbr = 0;
+    best = ~0ull;
+    if (P.count_bytes) ctr.blist += (uint64_t)nC * sizeof(R_t);
+    build_list<Wt>(brec, L, nL, m.C, nC, next_id, g.kV, cmap, g.u_off, g.u_adj, m.s_off, m.s_start);
+    // group twins (not in list mode: its R' lists need one entry per candidate)
+    if (P.group && !P.list && nC > 1) {
+      len = merge_twins<Wt>(m, brec, nC, lds_top, hbm_top, best, nbr, P.dom_skip != 0);
+    }
+    if (len == nC) {
+      // first push: the smallest rep
+      for (uint32_t i = lane; i < len; i += kWave) {
+        const uint32_t rp = brec[i].rep;
+        if (rp != kNone) {
+          const uint64_t c = ((uint64_t)rp << 32) | i;
+          best = c < best ? c : best;
+        }
+      }
+      best = (wave_min_pair(best));
+    }
+  }
+  enumerate_list<Wt>(P, m, brec, len, nL, nC, sumR, nR, best, nbr, ctr, t0, share_ctx, gw);
 }
 
 // ---------------------------------------------------------------------------
@@ -2779,19 +3047,50 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
   phase(ctr, P.profile, 1, t0);
   // 2-hop counts
   int32_t* cmap = m.cmap;
-  const uint64_t root_edges = uni64(count_edges(L, nL, g.u_off, g.u_adj, cmap, m.bm0, m.bm1, m.s_off,
-                                                m.s_start));
-  if (P.count_bytes) {
-    ctr.balg += 4ull * (sdeg + root_edges);
-    ctr.blist += 4ull * (sdeg + root_edges);
+  TileOut to{kTileNone, 0, 0, 0, 0, 0, 0, ~0ull, 0};
+  if constexpr (WMAX <= kMainW) {
+    // a top-level vertex with at most 32 neighbours: its grouped root list in one
+    // pass (tile_root).  The runs that need every candidate by itself (lists of
+    // bicliques, byte counts, recomputed children, no twin groups) and unordered
+    // lists take the general way.
+    if (k == 1 && nL > 1 && nL <= 32 && P.group && P.dom_skip && P.share && !P.recompute && !P.list &&
+        !P.count_bytes && g.nV < kSkip && m.lds_bytes >= kTileLds &&
+        m.arena_bytes >= kTileGroups * sizeof(Rec<1>)) {
+      to = tile_root(L, nL, g.u_off, g.u_adj, g.kV, g.nV, vk, m.lds, m.lds_bytes, m.fr_lds, m.s_off,
+                     m.s_start, (Rec<1>*)m.arena);
+      to.state = uni(to.state);
+      to.nR = uni(to.nR);
+      to.nC = uni(to.nC);
+      to.next_id = uni(to.next_id);
+      to.len = uni(to.len);
+      to.nbr = uni(to.nbr);
+      to.edges = uni(to.edges);
+      to.best = uni64(to.best);
+      to.sumR = uni64(to.sumR);
+    }
+  }
+  const bool tiled = to.state != kTileNone;
+  uint32_t nU2 = 0, nR = to.nR, nC = to.nC, next_id = to.next_id;
+  uint64_t root_edges = to.edges;
+  if (!tiled) {
+    root_edges = uni64(count_edges(L, nL, g.u_off, g.u_adj, cmap, m.bm0, m.bm1, m.s_off, m.s_start));
+    if (P.count_bytes) {
+      ctr.balg += 4ull * (sdeg + root_edges);
+      ctr.blist += 4ull * (sdeg + root_edges);
+    }
+    phase(ctr, P.profile, 2, t0);
+    const RootOut ro = split_two_hop(cmap, m.bm0, m.bm1, P.w.nW1, m.U, m.R, m.C, nL, vk);
+    nU2 = uni(ro.nU2);
+    nR = uni(ro.nR);
+    nC = uni(ro.nC);
+    next_id = uni(ro.next_id);
   }
   ctr.edges += root_edges;
-  phase(ctr, P.profile, 2, t0);
-  const RootOut ro = split_two_hop(cmap, m.bm0, m.bm1, P.w.nW1, m.U, m.R, m.C, nL, vk);
-  const uint32_t nU2 = uni(ro.nU2), nR = uni(ro.nR), nC = uni(ro.nC), next_id = uni(ro.next_id);
   // canonicity
   bool canonical;
-  if (k == 1) {
+  if (tiled) {
+    canonical = to.state == kTileList;
+  } else if (k == 1) {
     canonical = nR > 0 && m.R[0] == vk;
   } else {
     // every w in R below vk outside the prefix must contain the prefix's L
@@ -2829,9 +3128,10 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
   auto count_root = [&](uint64_t& sumL, uint64_t& sumR) {
     uint64_t sl = 0, sr = 0;
     for (uint32_t j = lane; j < nL; j += kWave) sl += g.kU[L[j]];
-    for (uint32_t i = lane; i < nR; i += kWave) sr += g.kV[m.R[i]];
+    if (!tiled)
+      for (uint32_t i = lane; i < nR; i += kWave) sr += g.kV[m.R[i]];
     sumL = uni64(wave_sum64(sl));
-    sumR = uni64(wave_sum64(sr));
+    sumR = tiled ? to.sumR : uni64(wave_sum64(sr));
     add_biclique(ctr, biclique_hash(sumL, sumR, g.swapped));
     if (P.list) {
       uint64_t at = list_reserve(P, 2ull + nL + nR);
@@ -2927,23 +3227,23 @@ __device__ __forceinline__ void run_task(const Params& P, const WaveMem& m, cons
   }
   count_root(sumL, sumR);
   // candidate index map: cmap[C[i]] = -(i+1), cmap[R[i]] = 0
-  for (uint32_t i = lane; i < nR; i += kWave) st_wg(cmap + m.R[i], 0);
-  for (uint32_t i = lane; i < nC; i += kWave) {
-    st_wg(cmap + m.C[i], -(int32_t)(i + 1));
+  if (!tiled) {
+    for (uint32_t i = lane; i < nR; i += kWave) st_wg(cmap + m.R[i], 0);
+    for (uint32_t i = lane; i < nC; i += kWave) st_wg(cmap + m.C[i], -(int32_t)(i + 1));
   }
   for (uint32_t j = lane; j < nL; j += kWave) {
     m.kL[j] = g.kU[L[j]];
     if (P.list) m.T[j] = L[j];
   }
   if (W <= 1) {
-    enumerate_task<1>(P, m, L, nL, nC, next_id, sumR, nR, ctr, t0, share_ctx, gw);
+    enumerate_task<1>(P, m, L, nL, nC, next_id, sumR, nR, to, ctr, t0, share_ctx, gw);
   } else if (W <= 2) {
-    enumerate_task<2>(P, m, L, nL, nC, next_id, sumR, nR, ctr, t0, share_ctx, gw);
+    enumerate_task<2>(P, m, L, nL, nC, next_id, sumR, nR, to, ctr, t0, share_ctx, gw);
   } else if (W <= 4) {
-    enumerate_task<4>(P, m, L, nL, nC, next_id, sumR, nR, ctr, t0, share_ctx, gw);
+    enumerate_task<4>(P, m, L, nL, nC, next_id, sumR, nR, to, ctr, t0, share_ctx, gw);
   } else if constexpr (WMAX >= 16) {
-    if (W <= 8) enumerate_task<8>(P, m, L, nL, nC, next_id, sumR, nR, ctr, t0, share_ctx, gw);
-    else enumerate_task<16>(P, m, L, nL, nC, next_id, sumR, nR, ctr, t0, share_ctx, gw);
+    if (W <= 8) enumerate_task<8>(P, m, L, nL, nC, next_id, sumR, nR, to, ctr, t0, share_ctx, gw);
+    else enumerate_task<16>(P, m, L, nL, nC, next_id, sumR, nR, to, ctr, t0, share_ctx, gw);
   }
 }
 
