@@ -41,8 +41,8 @@ enum CtlSlot { C_ROOT_NEXT = 0, C_WORK_LEFT, C_LIST_CURSOR, C_DEFERRED, C_WIDE_N
                C_QCTL = 8, C_IDLE = C_QCTL + 2 * mbe::kShards,
                C_NSLOTS = C_IDLE + mbe::kIdleWords * mbe::kIdleStride / mbe::kCtlStride };
 constexpr uint64_t kCtlWords = (uint64_t)C_NSLOTS * mbe::kCtlStride;
-// The waves' mail words follow (each wave clears its own before it waits).
-constexpr uint64_t kMailWords = (uint64_t)mbe::kIdleWords * 64 * mbe::kIdleStride;
+// The waves' mail boxes follow (each wave clears its own before it waits).
+constexpr uint64_t kMailWords = (uint64_t)mbe::kIdleWords * 64 * mbe::kMailStride;
 
 typedef void (*KernelFn)(mbe::Params);
 struct KernelChoice {

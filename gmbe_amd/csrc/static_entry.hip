@@ -114,7 +114,7 @@ static int execute_static_impl(const gmbe_graph* g, int bound_height, int bound_
   const uint64_t b_graph = o;  // what the host copies in
   const uint64_t o_kU = take(nU * 8), o_kV = take(nV * 8);
   const uint64_t o_gt = take(sizeof(mbe::DevGraph));
-  const uint64_t o_ctl = take((kCtlWords + kMailWords) * 8), o_acc = take(mbe::A_COUNT * 8);
+  const uint64_t o_ctl = take((kCtlWords + kStaticWaves * mbe::kMailStride) * 8), o_acc = take(mbe::A_COUNT * 8);
   const uint64_t o_q = take(kStaticQcap * mbe::kShards * mbe::kEntryWords * 4);
   const uint64_t o_qseq = take(kStaticQcap * mbe::kShards * 8);
   const uint64_t o_def = take(kStaticDeferred * sizeof(mbe::Task));
